@@ -144,6 +144,62 @@ __device__ __forceinline__ bf16x8_t rows_transposed(const unsigned char* l, int 
                                                  __builtin_bit_cast(uint2, a1).x, __builtin_bit_cast(uint2, a1).y));
 }
 
+// rows_transposed for every tile t of a chunk.  The reads and the wait for them
+// are one asm block: the compiler cannot tell which LDS bytes a transposing read
+// touches and makes its builtin wait for every buffer_load ... lds in flight,
+// also those of chunks to come; here only the caller's own wait for this chunk's
+// loads stands.  Tile t's address is tile 0's with t in bits 5 and up flipped
+// (the swizzle is an XOR of segment numbers).
+template <int D>
+__device__ __forceinline__ void rows_transposed_all(const unsigned char* l, int q4, int c16,
+                                                    bf16x8_t (&vt)[MfShape<D>::NT]) {
+  using S = MfShape<D>;
+  const int vkey = 4 * q4 + (c16 >> 2);
+  const uint32_t a0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_ptr)l)) + vkey * S::ROW +
+                      ((((c16 & 3) >> 1) ^ mf_swz<D>(vkey)) << 4) + (c16 & 1) * 8;
+  uint2 lo[S::NT], hi[S::NT];
+  if constexpr (D == 128) {
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %16\n\tds_read_b64_tr_b16 %8, %16 offset:4096\n\t"
+        "ds_read_b64_tr_b16 %1, %17\n\tds_read_b64_tr_b16 %9, %17 offset:4096\n\t"
+        "ds_read_b64_tr_b16 %2, %18\n\tds_read_b64_tr_b16 %10, %18 offset:4096\n\t"
+        "ds_read_b64_tr_b16 %3, %19\n\tds_read_b64_tr_b16 %11, %19 offset:4096\n\t"
+        "ds_read_b64_tr_b16 %4, %20\n\tds_read_b64_tr_b16 %12, %20 offset:4096\n\t"
+        "ds_read_b64_tr_b16 %5, %21\n\tds_read_b64_tr_b16 %13, %21 offset:4096\n\t"
+        "ds_read_b64_tr_b16 %6, %22\n\tds_read_b64_tr_b16 %14, %22 offset:4096\n\t"
+        "ds_read_b64_tr_b16 %7, %23\n\tds_read_b64_tr_b16 %15, %23 offset:4096\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(lo[0]), "=&v"(lo[1]), "=&v"(lo[2]), "=&v"(lo[3]), "=&v"(lo[4]), "=&v"(lo[5]), "=&v"(lo[6]),
+          "=&v"(lo[7]), "=&v"(hi[0]), "=&v"(hi[1]), "=&v"(hi[2]), "=&v"(hi[3]), "=&v"(hi[4]), "=&v"(hi[5]),
+          "=&v"(hi[6]), "=&v"(hi[7])
+        : "v"(a0), "v"(a0 ^ 32u), "v"(a0 ^ 64u), "v"(a0 ^ 96u), "v"(a0 ^ 128u), "v"(a0 ^ 160u), "v"(a0 ^ 192u),
+          "v"(a0 ^ 224u)
+        : "memory");
+  } else {
+    asm volatile(
+        "ds_read_b64_tr_b16 %0, %8\n\tds_read_b64_tr_b16 %4, %8 offset:2048\n\t"
+        "ds_read_b64_tr_b16 %1, %9\n\tds_read_b64_tr_b16 %5, %9 offset:2048\n\t"
+        "ds_read_b64_tr_b16 %2, %10\n\tds_read_b64_tr_b16 %6, %10 offset:2048\n\t"
+        "ds_read_b64_tr_b16 %3, %11\n\tds_read_b64_tr_b16 %7, %11 offset:2048\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(lo[0]), "=&v"(lo[1]), "=&v"(lo[2]), "=&v"(lo[3]), "=&v"(hi[0]), "=&v"(hi[1]), "=&v"(hi[2]),
+          "=&v"(hi[3])
+        : "v"(a0), "v"(a0 ^ 32u), "v"(a0 ^ 64u), "v"(a0 ^ 96u)
+        : "memory");
+  }
+#pragma unroll
+  for (int t = 0; t < S::NT; ++t)
+    vt[t] = __builtin_bit_cast(bf16x8_t, make_uint4(lo[t].x, lo[t].y, hi[t].x, hi[t].y));
+}
+
+// Block barrier that leaves N of this wave's newest buffer loads in flight
+// (__syncthreads() waits for all of them).  The wave's own LDS reads are done
+// before it.
+template <int N>
+__device__ __forceinline__ void barrier_keep_loads() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
 // s_waitcnt encodings (gfx9): vmcnt(0) alone, lgkmcnt(0) alone; vmcnt(N) for
 // N < 16 is kWaitVmBase | N.
 constexpr int kWaitVm0 = 0x0F70;

@@ -1,0 +1,44 @@
+"""The tiled block-granular attention (blocks of 32 keys and more) at the edges of
+its tiles: query vectors that fill no tile, a last block of few rows, lists longer
+than one 64-entry window, repeated and future blocks, rows with nothing to attend."""
+
+import numpy as np
+import pytest
+import torch
+
+from tests.helpers import f32, randn
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("d,g,n,bs,nkb,i64", [
+    (128, 1, 97, 32, 2, True),      # one partly filled tile, a last block of one row
+    (128, 3, 200, 32, 5, False),    # 96 query vectors: the second tile half used
+    (64, 7, 385, 64, 7, True),      # rows split over waves mid-group
+    (128, 8, 513, 256, 3, False),   # 2048 query vectors a block, a last block of one row
+    (64, 4, 2500, 32, 79, True),    # two list windows
+    (128, 2, 130, 128, 1, False)])  # a list without the rows' own block
+def test_block_tiles_vs_oracle(dev, orc, d, g, n, bs, nkb, i64):
+    from ssa_amd import kernels
+
+    B, h_kv = 1, 2
+    q = randn((B, n, h_kv * g, d), 91, torch.bfloat16)
+    k = randn((B, n, h_kv, d), 92, torch.bfloat16)
+    v = randn((B, n, h_kv, d), 93, torch.bfloat16)
+    nb = (n + bs - 1) // bs
+    gen = torch.Generator().manual_seed(94)
+    blocks = torch.stack([torch.randperm(nb, generator=gen)[:nkb] for _ in range(B * nb * h_kv)])
+    blocks = blocks.view(B, nb, h_kv, -1)
+    if nkb == 1:
+        blocks[:] = nb - 1           # the first block's rows have no key at all: zeros
+    elif nkb > 2:
+        blocks[..., 0] = blocks[..., 1]  # a block listed twice counts twice
+    blocks = blocks if i64 else blocks.to(torch.int32)
+    out = torch.empty(B, n, h_kv * g, d, device=dev, dtype=torch.float32)
+    flag = torch.zeros(1, dtype=torch.int32, device=dev)
+    kernels.block_sparse_attention(q.to(dev), k.to(dev), v.to(dev), blocks.to(dev), bs, out=out, error_flag=flag)
+    assert int(flag.item()) == 0
+    ref = orc.block_sparse_attention64(f32(q[0]), f32(k[0]), f32(v[0]), blocks[0].numpy(), bs)
+    np.testing.assert_allclose(out[0].cpu().numpy(), ref, rtol=1e-3, atol=1e-3)
+    bf = kernels.block_sparse_attention(q.to(dev), k.to(dev), v.to(dev), blocks.to(dev), bs)
+    assert torch.equal(bf, out.to(torch.bfloat16)), "bf16 output must be the fp32 output rounded"
