@@ -1401,6 +1401,302 @@ __global__ __launch_bounds__(64 * kSplitWaves) void sparse_attention_split_kerne
   }
 }
 
+// ---- fp32, selections that hold a good part of the keys -----------------------
+//
+// A row that selects top_k of n keys with n / top_k small shares most keys with
+// every other row, so gathering them row by row moves the same K and V rows once
+// per row.  Here one block takes 16 QT query vectors (R = 16 QT / g rows, all
+// their heads) and runs them against the keys in order, 16 at a time, with the
+// rows' selections as counts in LDS (KeyWindow; a tile no row of the block
+// selects is skipped):
+//   split      wave w of the block's four takes the tiles 4i + w, each with its
+//              own online softmax over all query vectors, and their states are
+//              combined at the end: a call of this size has few blocks, and a
+//              tile's K and V rows are read once per block;
+//   operands   K and V go from global memory straight to registers, V with the
+//              feature order of the output permuted so that each lane's piece is
+//              a float4 of one row (tile t, operand row r: feature 4r + t % 4 +
+//              64 (t / 4)); the q rows are in LDS;
+//   products   both on the fp32 matrix cores, whose 16x16x4 products are fmaf
+//              chains in ascending order, bit for bit; P needs no exchange between
+//              lanes (lane (q4, c16) holds keys 4 q4 + e of query c16, and step e
+//              of P.V takes keys {4 q4 + e});
+//   non-finite a V row with an infinity or NaN must not reach the rows that did
+//              not select it through 0 * inf: such a tile goes key by key.
+// Bound by the fp32 matrix cores' chains at one or two waves per SIMD: n = 2048 =
+// top_k, 8/2 heads, d = 64 takes 142 us (61 TFLOP/s) against 537 us row by row.
+constexpr int kDnWaves = 4;
+constexpr int kDnCountBytes = 40 << 10;  // LDS for the counts of one window
+
+template <int D, int QT>
+struct DnShape {
+  static constexpr int QV = 16 * QT;
+  static constexpr int QROW = D + 4;  // floats: rows start 4 banks apart
+  static constexpr int PROW = D + 4;  // state of a query vector: O, max, sum
+  static constexpr size_t q_bytes = sizeof(float) * QV * QROW;
+  static constexpr size_t part_bytes = sizeof(float) * kDnWaves * QV * PROW;
+  static size_t lds(int rows, int window) {
+    const size_t w = sizeof(uint16_t) * static_cast<size_t>(rows) * key_window_stride(window) +
+                     sizeof(uint32_t) * (window / kKeyTile / 32 + 1) + sizeof(uint16_t) * (window / kKeyTile + 8);
+    return align_up(q_bytes, 16) + (w > part_bytes ? align_up(w, 16) : part_bytes);
+  }
+};
+
+template <int D, int QT>
+__global__ __launch_bounds__(64 * kDnWaves, 2) void dense_f32_kernel(AttParams p, int window) {
+  using DS = DnShape<D, QT>;
+  constexpr int KB = D / 16, NT = D / 16, VQ = D / 64;
+  extern __shared__ __align__(16) unsigned char dn_lds[];
+  __shared__ int64_t s_pos[DS::QV], s_row[DS::QV];  // per row: key position (-1: no row), query row
+  const int g = p.g, R = DS::QV / g;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int q4 = lane >> 4, c16 = lane & 15;
+  const int64_t per_bh = udiv32(p.n_q + R - 1, R);
+  const int64_t bh = udiv32(blockIdx.x, per_bh);
+  const int64_t slot0 = (blockIdx.x - bh * per_bh) * R;
+  const int64_t bb = udiv32(bh, p.h_kv);
+  const int h = static_cast<int>(bh - bb * p.h_kv);
+  float* q_lds = reinterpret_cast<float*>(dn_lds);
+  unsigned char* rest = dn_lds + align_up(DS::q_bytes, 16);
+  KeyWindow kw;
+  kw.cnt = reinterpret_cast<uint32_t*>(rest);
+  kw.stride = key_window_stride(window);
+  const int cnt_words = R * kw.stride / 2, live_words = window / kKeyTile / 32 + 1;
+  kw.live = kw.cnt + cnt_words;
+  uint16_t* tiles = reinterpret_cast<uint16_t*>(kw.live + live_words) + wave * (window / kKeyTile / kDnWaves);
+
+  if (tid < R) {
+    AttRow ar{};
+    if (slot0 + tid < p.n_q) ar = att_row(p, bh * p.n_q + slot0 + tid);
+    s_pos[tid] = ar.ok ? ar.i : -1;
+    s_row[tid] = ar.ok ? ar.r : 0;
+  }
+  __syncthreads();
+  for (int e = tid; e < DS::QV * (D / 4); e += 64 * kDnWaves) {
+    const int qv = e / (D / 4), x = e - qv * (D / 4);
+    const int r = qv / g, hh = qv - r * g;
+    const bool ok = r < R && s_pos[r] >= 0;
+    const float* src = static_cast<const float*>(p.q) + bb * p.q_sb + (ok ? s_row[r] : 0) * p.q_sn +
+                       static_cast<int64_t>(h * g + (ok ? hh : 0)) * p.q_sh;
+    *reinterpret_cast<float4*>(q_lds + qv * DS::QROW + 4 * x) =
+        ok ? *reinterpret_cast<const float4*>(src + 4 * x) : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  const float* kbase = static_cast<const float*>(p.k) + bb * p.k_sb + static_cast<int64_t>(h) * p.k_sh;
+  const float* vbase = static_cast<const float*>(p.v) + bb * p.v_sb + static_cast<int64_t>(h) * p.v_sh;
+  int crow[QT];  // first count of the lane's query row
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) crow[qt] = min((16 * qt + c16) / g, R - 1) * kw.stride + 4 * q4;
+
+  float m_run[QT], l_run[QT];
+  floatx4_t oacc[QT][NT];
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    m_run[qt] = -INFINITY;
+    l_run[qt] = 0.0f;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) oacc[qt][t] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  for (int64_t w0 = 0; w0 < p.n; w0 += window) {
+    kw.key0 = w0;
+    kw.len = static_cast<int>(min(static_cast<int64_t>(window), p.n - w0));
+    __syncthreads();
+    for (int e = tid; e < cnt_words + live_words; e += 64 * kDnWaves) kw.cnt[e] = 0u;
+    __syncthreads();
+    for (int r = wave; r < R; r += kDnWaves) {
+      const int64_t pos = s_pos[r];
+      if (pos < 0) continue;
+      const int64_t ib = bb * p.idx_sb + s_row[r] * p.idx_sn + static_cast<int64_t>(h) * p.idx_sh;
+      auto load = [&](int64_t e) -> int64_t {
+        return p.idx_i64 ? static_cast<const int64_t*>(p.idx)[ib + e]
+                         : static_cast<int64_t>(static_cast<const int32_t*>(p.idx)[ib + e]);
+      };
+      strided_batches<4, 64>(p.top_k, lane, load, [&](int64_t, int64_t j) {
+        if (j < 0 || j >= p.n) {
+          if (p.err) p.err[0] = 1;
+        } else if (!(p.causal && j > pos)) {
+          kw.mark(r, j);
+        }
+      });
+    }
+    __syncthreads();
+    const int nlive = list_live_tiles<kDnWaves>(kw.live, static_cast<int>(ceil_div(kw.len, kKeyTile)), tiles, wave, lane);
+    float4 kf[KB], vf[4][VQ];
+    auto load_tile = [&](int t, float4 (&kd)[KB], float4 (&vd)[4][VQ]) {
+      const int64_t j0 = w0 + static_cast<int64_t>(t) * kKeyTile;
+      const int64_t jk = min(j0 + c16, p.n - 1);  // (past n: count 0)
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb)
+        kd[kb] = *reinterpret_cast<const float4*>(kbase + jk * p.k_sn + 16 * kb + 4 * q4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int64_t jv = min(j0 + 4 * q4 + e, p.n - 1);
+#pragma unroll
+        for (int y = 0; y < VQ; ++y)
+          vd[e][y] = *reinterpret_cast<const float4*>(vbase + jv * p.v_sn + 64 * y + 4 * c16);
+      }
+    };
+    int tile = nlive > 0 ? tiles[0] : 0;
+    if (nlive > 0) load_tile(tile, kf, vf);
+    for (int u = 0; u < nlive; ++u) {
+      const int tnext = u + 1 < nlive ? tiles[u + 1] : tile;
+      float sc[QT][4];
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+        floatx4_t s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+          const float4 qv = *reinterpret_cast<const float4*>(q_lds + (16 * qt + c16) * DS::QROW + 16 * kb + 4 * q4);
+          s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[kb].x, qv.x, s, 0, 0, 0);
+          s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[kb].y, qv.y, s, 0, 0, 0);
+          s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[kb].z, qv.z, s, 0, 0, 0);
+          s = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[kb].w, qv.w, s, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sc[qt][e] = s[e] * p.qk_scale_log2;
+      }
+      float4 vcur[4][VQ];
+      bool odd = false;  // some V value is not finite
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int y = 0; y < VQ; ++y) {
+          vcur[e][y] = vf[e][y];
+          odd |= !(isfinite(vf[e][y].x) && isfinite(vf[e][y].y) && isfinite(vf[e][y].z) && isfinite(vf[e][y].w));
+        }
+      const bool slow = __ballot(odd) != 0ull;
+      if (u + 1 < nlive) load_tile(tnext, kf, vf);
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+        const uint2 c2 = *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(kw.cnt) + crow[qt] +
+                                                         tile * kKeyTile);
+        const uint32_t cn[4] = {c2.x & 0xFFFFu, c2.x >> 16, c2.y & 0xFFFFu, c2.y >> 16};
+        float mx = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          sc[qt][e] = cn[e] ? sc[qt][e] : -INFINITY;
+          mx = fmaxf(mx, sc[qt][e]);
+        }
+        mx = rows4_reduce(mx, [](float a, float b) { return fmaxf(a, b); });
+        const float mnew = fmaxf(m_run[qt], mx);
+        const bool dead = mnew == -INFINITY;
+        const float alpha = dead ? 1.0f : exp2f(m_run[qt] - mnew);
+        m_run[qt] = mnew;
+        float pr[4], ps = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          pr[e] = (dead || !cn[e]) ? 0.0f : exp2f(sc[qt][e] - mnew) * static_cast<float>(cn[e]);
+          ps += pr[e];
+        }
+        l_run[qt] = l_run[qt] * alpha + ps;
+        if (__ballot(alpha != 1.0f)) {
+#pragma unroll
+          for (int t = 0; t < NT; ++t) oacc[qt][t] *= alpha;
+        }
+        if (!slow) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+              const float4 v4 = vcur[e][t / 4];
+              const float a = (t & 3) == 0 ? v4.x : (t & 3) == 1 ? v4.y : (t & 3) == 2 ? v4.z : v4.w;
+              oacc[qt][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, pr[e], oacc[qt][t], 0, 0, 0);
+            }
+        } else {
+          for (int x = 0; x < kKeyTile; ++x) {
+            const int src = (x >> 2) * 16 + c16;
+            const float pe = (x & 3) == 0 ? pr[0] : (x & 3) == 1 ? pr[1] : (x & 3) == 2 ? pr[2] : pr[3];
+            const uint32_t ce = (x & 3) == 0 ? cn[0] : (x & 3) == 1 ? cn[1] : (x & 3) == 2 ? cn[2] : cn[3];
+            const float pj = __shfl(pe, src);
+            const bool on = __shfl(static_cast<int>(ce), src) != 0;
+            const float* vr = vbase + min(w0 + static_cast<int64_t>(tile) * kKeyTile + x, p.n - 1) * p.v_sn;
+            if (on) {
+#pragma unroll
+              for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                  oacc[qt][t][e] = fma_rn(pj, vr[4 * (4 * q4 + e) + (t & 3) + 64 * (t / 4)], oacc[qt][t][e]);
+            }
+          }
+        }
+      }
+      tile = tnext;
+    }
+  }
+
+  // The waves' states: O, running max and sum per query vector.
+  __syncthreads();
+  float* part = reinterpret_cast<float*>(rest);
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    const float lt = rows4_reduce(l_run[qt], [](float a, float b) { return a + b; });
+    float* pp = part + (wave * DS::QV + 16 * qt + c16) * DS::PROW;
+    // lane (q4, c16): features 4 (4 q4 + e) + t % 4 + 64 (t / 4), four at a time
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int y = 0; y < VQ; ++y)
+        *reinterpret_cast<float4*>(pp + 64 * y + 4 * (4 * q4 + e)) =
+            make_float4(oacc[qt][4 * y][e], oacc[qt][4 * y + 1][e], oacc[qt][4 * y + 2][e], oacc[qt][4 * y + 3][e]);
+    if (q4 == 0) {
+      pp[D] = m_run[qt];
+      pp[D + 1] = lt;
+    }
+  }
+  __syncthreads();
+  for (int e = tid; e < R * g * (D / 4); e += 64 * kDnWaves) {
+    const int qv = e / (D / 4), x = e - qv * (D / 4);
+    const int r = qv / g, hh = qv - r * g;
+    if (s_pos[r] < 0) continue;
+    float M = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kDnWaves; ++w) M = fmaxf(M, part[(w * DS::QV + qv) * DS::PROW + D]);
+    float L = 0.0f;
+    float4 O = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int w = 0; w < kDnWaves; ++w) {
+      const float* pp = part + (w * DS::QV + qv) * DS::PROW;
+      if (pp[D] == -INFINITY) continue;  // no selected key in this wave's tiles
+      const float a = exp2f(pp[D] - M);
+      L += a * pp[D + 1];
+      const float4 o4 = *reinterpret_cast<const float4*>(pp + 4 * x);
+      O.x += a * o4.x; O.y += a * o4.y; O.z += a * o4.z; O.w += a * o4.w;
+    }
+    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+    const int64_t ob = bb * p.o_sb + s_row[r] * p.o_sn + static_cast<int64_t>(h * g + hh) * p.o_sh + 4 * x;
+    if (p.out_bf16)
+      *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.out) + ob) =
+          make_uint2(pack_bf16x2(O.x * inv, O.y * inv), pack_bf16x2(O.z * inv, O.w * inv));
+    else
+      *reinterpret_cast<float4*>(static_cast<float*>(p.out) + ob) =
+          make_float4(O.x * inv, O.y * inv, O.z * inv, O.w * inv);
+  }
+}
+
+// Taken while n * max(g, 2) <= 16 top_k: its time grows with n g, the row
+// kernel's with top_k (a row's products cost the same for 1 to 4 heads there).
+// Random selections on MI355X, us, row kernel / this one:
+//   d = 64   8 kv heads, g = 1:  n = 2048, k = 512: 453 / 222;  k = 256: 238 / 165;  k = 128: 131 / 144
+//            2 kv heads, g = 4:  n = 2048, k = 2048: 657 / 143;  k = 512: 152 / 115;  k = 256: 79 / 112
+//            2 kv heads, g = 8:  n = 2048, k = 2048: 652 / 242;  k = 512: 164 / 219
+//   d = 128  2 kv heads, g = 4:  n = 2048, k = 2048: 1369 / 255;  k = 512: 341 / 237;  k = 256: 184 / 231
+// Two 16-query tiles a block at d = 64 once that leaves 512 blocks (2 waves a
+// SIMD); at d = 128 two do not fit the registers.
+constexpr int kDnKeysPerSlot = 16;
+constexpr int64_t kDnTwoTiles = 32 * 512;  // query vectors
+
+template <int D, int QT>
+int launch_dense_f32(const AttParams& p, hipStream_t st) {
+  using DS = DnShape<D, QT>;
+  const int R = DS::QV / p.g;
+  const int window = key_window(p.n, R, kDnCountBytes);
+  const size_t lds = DS::lds(R, window);
+  if (int s = reserve_lds(reinterpret_cast<const void*>(dense_f32_kernel<D, QT>), lds, "dense_f32_kernel")) return s;
+  const int64_t blocks = (p.rows / p.n_q) * ceil_div(p.n_q, R);
+  dense_f32_kernel<D, QT><<<dim3(static_cast<unsigned>(blocks)), 64 * kDnWaves, lds, st>>>(p, window);
+  return check_launch("dense_f32_kernel");
+}
+
 template <typename T, int D>
 int launch_att_d(const AttParams& p, hipStream_t st) {
   const int64_t blocks = ceil_div(p.rows, kAttWaves);
@@ -1442,6 +1738,13 @@ int launch_att_d(const AttParams& p, hipStream_t st) {
       if (p.blk_log2 > 0) sparse_attention_mfma_kernel<D, true><<<grid, 64 * kMfWaves, 0, st>>>(pr);
       else sparse_attention_mfma_kernel<D, false><<<grid, 64 * kMfWaves, 0, st>>>(pr);
       return check_launch("sparse_attention_mfma_kernel");
+    }
+  }
+  if constexpr (sizeof(T) == 4 && (D == 64 || D == 128)) {
+    if (p.blk_log2 == 0 && p.d == D && p.top_k < (1 << 16) && p.n * max(p.g, 2) <= static_cast<int64_t>(p.top_k) * kDnKeysPerSlot) {
+      const int64_t qvs = p.rows * p.g;
+      if (D == 64 && qvs >= kDnTwoTiles) return launch_dense_f32<D, (D == 64 ? 2 : 1)>(p, st);
+      return launch_dense_f32<D, 1>(p, st);
     }
   }
   if (p.g <= 4) sparse_attention_kernel<T, D, 4><<<dim3(static_cast<unsigned>(blocks)), kAttThreads, 0, st>>>(p);

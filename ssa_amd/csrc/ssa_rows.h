@@ -200,6 +200,63 @@ __device__ __forceinline__ void barrier_keep_loads() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
+// ---- key windows: how often each of a few rows selects each key ----------------
+//
+// The fp32 kernels that run many query vectors against consecutive keys
+// (dense_f32_kernel, dense_bwd_f32_kernel) read a row's selection as counts: cnt
+// holds 16 bits per (row, key) of a window of keys (slots of equal index count
+// once each, and top_k < 2^16), stride keys apart, and `live` a bit per 16-key
+// tile that some row selects.  Both are cleared before.
+constexpr int kKeyTile = 16;
+struct KeyWindow {
+  uint32_t* cnt;   // [rows][stride / 2], two keys a word
+  uint32_t* live;  // [ceil(window / kKeyTile / 32)]
+  int stride;      // keys, even
+  int64_t key0;
+  int len;
+  __device__ __forceinline__ void mark(int row, int64_t key) const {
+    const int64_t j = key - key0;
+    if (j < 0 || j >= len) return;
+    const int jw = static_cast<int>(j);
+    atomicAdd(&cnt[(row * stride + jw) >> 1], 1u << ((jw & 1) * 16));
+    const uint32_t bit = 1u << ((jw / kKeyTile) & 31);
+    uint32_t* w = &live[jw / kKeyTile / 32];
+    if (!(*w & bit)) atomicOr(w, bit);
+  }
+};
+
+// Keys of a window a block of R rows can count in `bytes` of LDS: a multiple of
+// 64, at least 64.
+__host__ __device__ inline int key_window(int64_t n, int rows, int bytes) {
+  const int fit = bytes / (2 * rows) / 64 * 64 - 64;
+  const int64_t all = (n + 63) / 64 * 64;
+  return static_cast<int>(all < fit ? all : (fit < 64 ? 64 : fit));
+}
+// Row stride of the counts: 8 keys past the window, so that the rows of one
+// read (4 keys each) start 4 banks apart.
+__host__ __device__ inline int key_window_stride(int window) { return window + 8; }
+
+// The live tiles among W w-th ones (w = wave, W = waves of the block) as a list
+// that the wave builds for itself, ceil(tiles / W) entries; returns their number.
+// Which wave takes a tile depends on the tile's number alone, so that a row's
+// sums do not depend on the rows it shares a block with (a tile it selects
+// nothing of adds zeros).  The marks are done before (barrier).
+template <int W>
+__device__ __forceinline__ int list_live_tiles(const uint32_t* live, int tiles, uint16_t* list, int wave, int lane) {
+  int base = 0;
+  for (int t0 = 0; W * t0 + wave < tiles; t0 += 64) {
+    const int t = W * (t0 + lane) + wave;
+    const bool on = t < tiles && ((live[t >> 5] >> (t & 31)) & 1u);
+    const uint64_t m = __ballot(on);
+    if (on) list[base + __popcll(m & ((1ull << lane) - 1))] = static_cast<uint16_t>(t);
+    base += __popcll(m);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  return __builtin_amdgcn_readfirstlane(base);
+}
+
 // s_waitcnt encodings (gfx9): vmcnt(0) alone, lgkmcnt(0) alone; vmcnt(N) for
 // N < 16 is kWaitVmBase | N.
 constexpr int kWaitVm0 = 0x0F70;

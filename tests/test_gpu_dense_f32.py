@@ -1,0 +1,86 @@
+"""fp32 attention over selections that hold a good part of the keys (key tiles with
+counts in LDS): several key windows, rows that fill no tile, repeated keys, dropped
+slots, a processing order and non-finite values of keys a row did not select."""
+
+import numpy as np
+import pytest
+import torch
+
+from tests.helpers import f32, randn
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(n, h_kv, g, d, k, seed):
+    q, kk, v = randn((1, n, h_kv * g, d), seed), randn((1, n, h_kv, d), seed + 1), randn((1, n, h_kv, d), seed + 2)
+    gen = torch.Generator().manual_seed(seed + 3)
+    idx = torch.stack([torch.randperm(n, generator=gen)[:k] for _ in range(n * h_kv)]).view(1, n, h_kv, k)
+    return q, kk, v, idx
+
+
+@pytest.mark.parametrize("d,g,h_kv,n,k,causal,i64", [
+    (64, 1, 2, 1999, 300, False, True),    # 16 rows a block, four key windows
+    (64, 3, 2, 331, 70, True, False),      # 15 of 16 query vectors used
+    (64, 4, 4, 1100, 300, True, True),     # two query tiles a block
+    (128, 5, 1, 257, 100, True, True),
+    (128, 16, 1, 40, 40, False, False),    # one row a block, all keys
+    (64, 8, 1, 17, 30, False, True)])      # k > n: padded with key 0
+def test_dense_f32_vs_oracle(dev, orc, d, g, h_kv, n, k, causal, i64):
+    from ssa_amd import kernels
+
+    q, kk, v, idx = _case(n, h_kv, g, d, min(k, n), 21)
+    if k > n:
+        idx = torch.cat((idx, idx.new_zeros(1, n, h_kv, k - n)), dim=-1)
+    elif k < n:
+        idx[..., 1] = idx[..., 0]  # counts twice
+    idx = idx if i64 else idx.to(torch.int32)
+    flag = torch.zeros(1, dtype=torch.int32, device=dev)
+    order = torch.stack([torch.randperm(n) for _ in range(h_kv)]).to(torch.int32)[None]
+    got = kernels.sparse_attention(q.to(dev), kk.to(dev), v.to(dev), idx.to(dev), None, causal, error_flag=flag)
+    other = kernels.sparse_attention(q.to(dev), kk.to(dev), v.to(dev), idx.to(dev), None, causal,
+                                     row_order=order.to(dev))
+    assert int(flag.item()) == 0
+    assert torch.equal(got, other), "a row's result must not depend on the rows it shares a block with"
+    ref = orc.sparse_attention(f32(q[0]), f32(kk[0]), f32(v[0]), idx[0].to(torch.int64).numpy(), causal=causal)
+    # 32-bit sums of at most n terms against 64 bits
+    np.testing.assert_allclose(got[0].cpu().numpy(), ref, rtol=1e-5, atol=1e-5)
+
+
+def test_dense_f32_non_finite_values_reach_their_rows_only(dev, orc):
+    from ssa_amd import kernels
+
+    n, h_kv, g, d, k = 96, 2, 4, 64, 48
+    q, kk, v, idx = _case(n, h_kv, g, d, k, 31)
+    v[0, 7, 0, 3] = float("inf")
+    v[0, 50, 1, 60] = float("nan")
+    kk[0, 20, 0, 0] = float("inf")
+    got = kernels.sparse_attention(q.to(dev), kk.to(dev), v.to(dev), idx.to(dev))[0].cpu()
+    has = torch.zeros(n, h_kv, n, dtype=torch.bool).scatter_(2, idx[0], True)
+    clean = got.isfinite().view(n, h_kv, g, d)
+    assert clean[~has[:, 0, 7] & ~has[:, 0, 20], 0].all() and clean[~has[:, 1, 50], 1].all()
+    rows = has[:, 1, 50]
+    assert not clean[rows, 1, :, 60].any() and clean[rows, 1, :, :60].all()
+
+
+def test_dense_f32_flags_and_order(dev):
+    from ssa_amd import kernels
+
+    n, h_kv, g, d, k = 64, 1, 4, 64, 32
+    q, kk, v, idx = _case(n, h_kv, g, d, k, 41)
+    good = kernels.sparse_attention(q.to(dev), kk.to(dev), v.to(dev), idx.to(dev))
+    bad = idx.clone()
+    bad[0, 5, 0, 9] = n
+    flag = torch.zeros(1, dtype=torch.int32, device=dev)
+    out = kernels.sparse_attention(q.to(dev), kk.to(dev), v.to(dev), bad.to(dev), error_flag=flag)
+    assert int(flag.item()) == 1
+    keep = torch.arange(n) != 5
+    assert torch.equal(out[0, keep], good[0, keep])
+    order = torch.arange(n, dtype=torch.int32)[None, None].clone()
+    order[0, 0, 9] = n                       # dropped: row 9 is never listed
+    part = torch.full_like(good, 7.0)
+    flag.zero_()
+    kernels.sparse_attention(q.to(dev), kk.to(dev), v.to(dev), idx.to(dev), out=part, error_flag=flag,
+                             row_order=order.to(dev))
+    assert int(flag.item()) == 1 and (part[0, 9] == 7.0).all()
+    keep = torch.arange(n) != 9
+    assert torch.equal(part[0, keep], good[0, keep])
