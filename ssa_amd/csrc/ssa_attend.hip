@@ -16,6 +16,8 @@
 #include "ssa_internal.h"
 #include "ssa_rows.h"
 
+#include <type_traits>
+
 namespace ssa {
 namespace {
 
@@ -887,8 +889,10 @@ sparse_attention_mfma_kernel(AttParams p) {
 // the running maximum and the exponent's fma when it is positive and finite
 // (max(s) c is the maximum of the scaled scores); otherwise the scores are
 // scaled first (cmul = 1).  The V^T fragments are read behind the score MFMAs,
-// which run meanwhile.
-template <int D, int QT, class Masked, class Keep>
+// which run meanwhile.  GUARD: a masked key's V may hold an infinity or NaN that
+// must not reach the queries it is masked for through 0 * inf; a chunk holding
+// one adds its keys one by one.
+template <int D, int QT, bool GUARD, class Masked, class Keep>
 __device__ __forceinline__ void dense_chunk(const unsigned char* kl, const unsigned char* vl, int q4, int c16, int kswz,
                                             const bf16x8_t (&qf)[QT][MfShape<D>::KB], float c, Masked masked,
                                             Keep keep, float (&m_run)[QT], float (&l_run)[QT],
@@ -918,6 +922,20 @@ __device__ __forceinline__ void dense_chunk(const unsigned char* kl, const unsig
   }
   bf16x8_t vt[S::NT];
   rows_transposed_all<D>(vl, q4, c16, vt);
+  bool slow = false;
+  if constexpr (GUARD) {
+    typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+    u16x2 top = {0, 0};
+#pragma unroll
+    for (int t = 0; t < S::NT; ++t) {
+      const uint4 w = __builtin_bit_cast(uint4, vt[t]);
+      top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, w.x & 0x7FFF7FFFu));
+      top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, w.y & 0x7FFF7FFFu));
+      top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, w.z & 0x7FFF7FFFu));
+      top = __builtin_elementwise_max(top, __builtin_bit_cast(u16x2, w.w & 0x7FFF7FFFu));
+    }
+    slow = __ballot(top.x >= 0x7F80u || top.y >= 0x7F80u) != 0ull;
+  }
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
     if (!cpos) {
@@ -958,6 +976,28 @@ __device__ __forceinline__ void dense_chunk(const unsigned char* kl, const unsig
     if (__ballot(alpha != 1.0f)) {
 #pragma unroll
       for (int t = 0; t < S::NT; ++t) oacc[qt][t] *= alpha;
+    }
+    if (GUARD && slow) {
+#pragma unroll 1
+      for (int key = 0; key < kMfChunk; ++key) {  // p of `key` is pr[4 (key / 16) + key % 4] of lane row key / 4 % 4
+        float mine = -1.0f;                       // -1: not attended
+#pragma unroll
+        for (int x = 0; x < 8; ++x)
+          if (x == 4 * (key >> 4) + (key & 3) && sc[qt][x] != -INFINITY) mine = pr[x];
+        const float pj = __shfl(mine, 16 * ((key >> 2) & 3) + c16);
+        const int off = key * S::ROW + (((q4 >> 1) ^ mf_swz<D>(key)) << 4) + (q4 & 1) * 8;
+#pragma unroll
+        for (int t = 0; t < S::NT; ++t) {
+          const uint2 w = *reinterpret_cast<const uint2*>(vl + (off ^ (t << 5)));
+          if (pj != -1.0f) {
+            oacc[qt][t][0] = fma_rn(pj, __uint_as_float(w.x << 16), oacc[qt][t][0]);
+            oacc[qt][t][1] = fma_rn(pj, __uint_as_float(w.x & 0xFFFF0000u), oacc[qt][t][1]);
+            oacc[qt][t][2] = fma_rn(pj, __uint_as_float(w.y << 16), oacc[qt][t][2]);
+            oacc[qt][t][3] = fma_rn(pj, __uint_as_float(w.y & 0xFFFF0000u), oacc[qt][t][3]);
+          }
+        }
+      }
+      continue;
     }
 #pragma unroll
     for (int t = 0; t < S::NT; ++t) {
@@ -1064,7 +1104,7 @@ __global__ __launch_bounds__(64 * kPfxWaves, 2) void prefix_attention_kernel(Att
   using S = MfShape<D>;
   constexpr int kLoadsPerWave = S::NLD / kPfxWaves;  // of K and of V, per chunk
   static_assert(S::NLD % kPfxWaves == 0, "chunk loads split evenly over the waves");
-  __shared__ __align__(16) unsigned char kv[kPfxBufs][2][kMfChunk * S::ROW];  // [buffer][K, V]
+  __shared__ __align__(256) unsigned char kv[kPfxBufs][2][kMfChunk * S::ROW];  // [buffer][K, V]
   __shared__ int s_x[kPfxQv];
   __shared__ int s_xmax;
   const int g = p.g;
@@ -1174,7 +1214,7 @@ __global__ __launch_bounds__(64 * kPfxWaves, 2) void prefix_attention_kernel(Att
     else barrier_keep_loads<0>();
     if (u + 2 < nch) issue(u + 2);
     const int jbase = u * kMfChunk + 4 * q4;
-    dense_chunk<D, 2>(
+    dense_chunk<D, 2, false>(
         kv[u % kPfxBufs][0], kv[u % kPfxBufs][1], q4, c16, kswz, qf, p.qk_scale_log2,
         [&](int qt) { return (u + 1) * kMfChunk > jfull[qt]; },
         [&](int qt, int x) { return jbase + x < xr[qt] && jbase + x <= ilim[qt]; }, m_run, l_run, oacc);
@@ -1227,7 +1267,7 @@ __global__ __launch_bounds__(64 * kBlkWaves, 2) void block_attention_kernel(AttP
   constexpr int kLoadsPerWave = S::NLD / kBlkWaves;  // of K and of V, per chunk
   static_assert(S::NLD % kBlkWaves == 0, "chunk loads split evenly over the waves");
   constexpr int kQv = 16 * QT * kBlkWaves;
-  __shared__ __align__(16) unsigned char kv[kPfxBufs][2][kMfChunk * S::ROW];  // [buffer][K, V]
+  __shared__ __align__(256) unsigned char kv[kPfxBufs][2][kMfChunk * S::ROW];  // [buffer][K, V]
   const int g = p.g, lg = p.blk_log2, bs = 1 << lg;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1302,54 +1342,59 @@ __global__ __launch_bounds__(64 * kBlkWaves, 2) void block_attention_kernel(AttP
   const int kswz = mf_swz<D>(c16);
   const int nlist = p.top_k >> lg;
   const int64_t ibase = bb * p.idx_sb + bq * p.idx_sn + static_cast<int64_t>(h) * p.idx_sh;
-  for (int w0 = 0; w0 < nlist; w0 += 64) {
-    // every wave reads the 64 entries by itself, one per lane, and walks the
-    // kept ones by their ballot bits (no LDS read, which would wait for the
-    // chunk loads in flight)
-    const int e = w0 + lane;
-    int64_t id = -1;
-    if (e < nlist)
-      id = p.idx_i64 ? static_cast<const int64_t*>(p.idx)[ibase + e]
-                     : static_cast<int64_t>(static_cast<const int32_t*>(p.idx)[ibase + e]);
-    if (e < nlist && (id < 0 || id >= p.nbk) && p.err) p.err[0] = 1;
-    uint64_t left = __ballot(id >= 0 && id <= bq);
-    const int nch = __popcll(left) * cpb;
-    if (nch == 0) continue;
-    const int id32 = static_cast<int>(id);
-    // first key of the chunk to be loaded next: block ids in list order
-    int cur = 0, part = cpb;
-    auto next_key = [&]() {
-      if (part == cpb) {
-        cur = lane_value(id32, __builtin_ctzll(left)) << lg;
-        left &= left - 1;
-        part = 0;
+  // the listed blocks of the past, then the query block itself where it is listed
+  auto attend = [&](auto own_tag) {
+    constexpr bool own = decltype(own_tag)::value;
+    for (int w0 = 0; w0 < nlist; w0 += 64) {
+      // every wave reads the 64 entries by itself, one per lane, and walks the
+      // kept ones by their ballot bits (no LDS read, which would wait for the
+      // chunk loads in flight)
+      const int e = w0 + lane;
+      int64_t id = -1;
+      if (e < nlist)
+        id = p.idx_i64 ? static_cast<const int64_t*>(p.idx)[ibase + e]
+                       : static_cast<int64_t>(static_cast<const int32_t*>(p.idx)[ibase + e]);
+      if (e < nlist && (id < 0 || id >= p.nbk) && p.err) p.err[0] = 1;
+      uint64_t left = __ballot(own ? id == bq : (id >= 0 && id < bq));
+      const int nch = __popcll(left) * cpb;
+      if (nch == 0) continue;
+      const int id32 = static_cast<int>(id);
+      // first key of the chunk to be loaded next: block ids in list order
+      int cur = 0, part = cpb;
+      auto next_key = [&]() {
+        if (part == cpb) {
+          cur = lane_value(id32, __builtin_ctzll(left)) << lg;
+          left &= left - 1;
+          part = 0;
+        }
+        return cur + kMfChunk * part++;
+      };
+      __syncthreads();  // every wave is done with the window before, no load is in flight
+      int j0 = next_key();
+      issue(0, j0);
+      int j1 = nch > 1 ? next_key() : 0;
+      if (nch > 1) issue(1, j1);
+      int b0 = 0, b2 = 2;
+      for (int u = 0; u < nch; ++u) {
+        if (u + 1 < nch) barrier_keep_loads<2 * kLoadsPerWave>();
+        else barrier_keep_loads<0>();
+        int j2 = 0;
+        if (u + 2 < nch) {
+          j2 = next_key();
+          issue(b2, j2);
+        }
+        dense_chunk<D, QT, own>(
+            kv[b0][0], kv[b0][1], q4, c16, kswz, qf, p.qk_scale_log2, [](int) { return own; },
+            [&](int qt, int x) { return j0 + 4 * q4 + x <= ilim[qt]; }, m_run, l_run, oacc);
+        j0 = j1;
+        j1 = j2;
+        b0 = b0 == kPfxBufs - 1 ? 0 : b0 + 1;
+        b2 = b2 == kPfxBufs - 1 ? 0 : b2 + 1;
       }
-      return cur + kMfChunk * part++;
-    };
-    __syncthreads();  // every wave is done with the window before, no load is in flight
-    int j0 = next_key();
-    issue(0, j0);
-    int j1 = nch > 1 ? next_key() : 0;
-    if (nch > 1) issue(1, j1);
-    int b0 = 0, b2 = 2;
-    for (int u = 0; u < nch; ++u) {
-      if (u + 1 < nch) barrier_keep_loads<2 * kLoadsPerWave>();
-      else barrier_keep_loads<0>();
-      int j2 = 0;
-      if (u + 2 < nch) {
-        j2 = next_key();
-        issue(b2, j2);
-      }
-      dense_chunk<D, QT>(
-          kv[b0][0], kv[b0][1], q4, c16, kswz, qf, p.qk_scale_log2,
-          [&](int) { return j0 >= static_cast<int>(r0); },
-          [&](int qt, int x) { return j0 + 4 * q4 + x <= ilim[qt]; }, m_run, l_run, oacc);
-      j0 = j1;
-      j1 = j2;
-      b0 = b0 == kPfxBufs - 1 ? 0 : b0 + 1;
-      b2 = b2 == kPfxBufs - 1 ? 0 : b2 + 1;
     }
-  }
+  };
+  attend(std::integral_constant<bool, false>{});
+  attend(std::integral_constant<bool, true>{});
 #pragma unroll
   for (int qt = 0; qt < QT; ++qt) {
     const float lt = rows4_reduce(l_run[qt], [](float a, float b) { return a + b; });

@@ -149,7 +149,7 @@ __device__ __forceinline__ bf16x8_t rows_transposed(const unsigned char* l, int 
 // touches and makes its builtin wait for every buffer_load ... lds in flight,
 // also those of chunks to come; here only the caller's own wait for this chunk's
 // loads stands.  Tile t's address is tile 0's with t in bits 5 and up flipped
-// (the swizzle is an XOR of segment numbers).
+// (the swizzle is an XOR of segment numbers), which wants l aligned to a row.
 template <int D>
 __device__ __forceinline__ void rows_transposed_all(const unsigned char* l, int q4, int c16,
                                                     bf16x8_t (&vt)[MfShape<D>::NT]) {

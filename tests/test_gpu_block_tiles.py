@@ -42,3 +42,23 @@ def test_block_tiles_vs_oracle(dev, orc, d, g, n, bs, nkb, i64):
     np.testing.assert_allclose(out[0].cpu().numpy(), ref, rtol=1e-3, atol=1e-3)
     bf = kernels.block_sparse_attention(q.to(dev), k.to(dev), v.to(dev), blocks.to(dev), bs)
     assert torch.equal(bf, out.to(torch.bfloat16)), "bf16 output must be the fp32 output rounded"
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_block_tiles_non_finite_value_stays_in_its_past(dev, d):
+    """A key that is still to come for a row of its own block must not reach that row."""
+    from ssa_amd import kernels
+
+    n, g, bs, at = 96, 4, 32, 45
+    q, k, v = (randn((1, n, h, d), 95 + h, torch.bfloat16) for h in (g, 1, 2))
+    v = v[:, :, :1].contiguous()
+    blocks = torch.arange(3).expand(3, 3).contiguous().view(1, 3, 1, 3)
+    good = kernels.block_sparse_attention(q.to(dev), k.to(dev), v.to(dev), blocks.to(dev), bs)
+    v[0, at, 0, 5] = float("inf")
+    got = kernels.block_sparse_attention(q.to(dev), k.to(dev), v.to(dev), blocks.to(dev), bs)
+    assert torch.equal(got[0, :32], good[0, :32])
+    # the rows before `at` in its block: key by key instead of in the matrix cores
+    torch.testing.assert_close(got[0, :at].float(), good[0, :at].float(), rtol=2 ** -7, atol=2 ** -9)
+    assert not got[0, at:, :, 5].isfinite().any()
+    rest = torch.arange(d) != 5
+    torch.testing.assert_close(got[0, at:][..., rest].float(), good[0, at:][..., rest].float(), rtol=2 ** -7, atol=2 ** -9)
