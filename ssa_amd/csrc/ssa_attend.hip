@@ -275,13 +275,6 @@ struct VSlice {
   }
 };
 
-// LDS hand-off between lanes of one wave (each wave owns its LDS slices).
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
 // Per chunk of kChunk selected keys (lanes < kChunk load the indices):
 //   K: kTiles tiles of 16 keys; lane (q4, c16) loads 16 B of key tile*16+c16
 //      per 32-dim block straight into the MFMA B fragment;

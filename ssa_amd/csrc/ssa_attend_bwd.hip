@@ -1506,6 +1506,434 @@ bucket_attention_bwd_kernel(BwdParams p, BucketParams bp) {
   }
 }
 
+// ---- fp32, selections that hold a good part of the keys -----------------------
+//
+// The forward's layout (dense_f32_kernel): one block takes 16 QT query vectors (R
+// = 16 QT / g rows, all their heads) against the keys in order, 16 at a time, the
+// selections as counts in LDS, wave w of four taking the tiles 4i + w that some
+// row selects.
+//   pass 1     S per tile, each wave's running max and sum per query vector,
+//              combined over the waves;
+//   pass 2     S^T = K Q^T and dP^T = V dO^T (lane (q4, c16): keys 4 q4 + e of query
+//              vector c16), p, ds = p (dP - D); dQ^T += K^T dS^T with step e taking
+//              keys {4 q4 + e}, so dS needs no exchange (K's features permuted as
+//              in the forward); P and dS pass through LDS to [query vector][key]
+//              for dV = P^T dO and dK = dS^T Q, summed over the block's QT tiles in
+//              registers and added to memory once per (key, feature) and block,
+//              where the row kernel adds them once per row.
+// All products are fp32 fmaf chains on the matrix cores.  Only what a row selects
+// may meet a value that is not finite (0 * inf): a K tile, or a block's q or dO,
+// that holds one goes key by key (dQ), query vector by query vector (dK, dV).
+// Bound by the matrix-core chains at two waves per SIMD and the fp32 atomics of dK
+// and dV.  The README layer (batch 2, n = 1024, 8/2 heads, d = 64, k = 256): 205 us
+// against 1121 us row by row, where 134 M atomics alone took about 0.4 ms.
+constexpr int kDbWaves = 4;
+constexpr int kDbCountBytes = 24 << 10;  // LDS for the counts of one window
+constexpr int kDbTr = 20;                // floats per transposed P / dS row
+
+template <int D, int QT>
+struct DbShape {
+  static constexpr int QV = 16 * QT;
+  static constexpr int ROW = D + 4;  // floats per q / dO row in LDS
+  static constexpr size_t qd_bytes = sizeof(float) * 2 * QV * ROW;
+  // per wave: P and dS as [query vector][key], then a [key][feature] tile on its way out
+  static constexpr int wave_floats = 2 * 16 * kDbTr > 16 * ROW ? 2 * 16 * kDbTr : 16 * ROW;
+  static constexpr size_t tr_bytes = sizeof(float) * kDbWaves * wave_floats;
+  static constexpr size_t part_bytes = sizeof(float) * kDbWaves * QV * ROW;  // dQ per wave, at the end
+  static size_t cnt_bytes(int rows, int window) {
+    return sizeof(uint16_t) * static_cast<size_t>(rows) * key_window_stride(window) +
+           sizeof(uint32_t) * (window / kKeyTile / 32 + 1) + sizeof(uint16_t) * (window / kKeyTile + 8);
+  }
+  static size_t lds(int rows, int window) {
+    const size_t loop = tr_bytes + align_up(cnt_bytes(rows, window), 16);
+    return qd_bytes + (loop > part_bytes ? loop : part_bytes);
+  }
+};
+
+template <int D, int QT>
+__global__ __launch_bounds__(64 * kDbWaves, 2) void dense_bwd_f32_kernel(BwdParams p, int window) {
+  using DS = DbShape<D, QT>;
+  constexpr int KB = D / 16, NT = D / 16, VQ = D / 64, NTH = 64 * kDbWaves;
+  extern __shared__ __align__(16) unsigned char db_lds[];
+  __shared__ int64_t s_row[DS::QV];                  // query row (= key position), -1: none
+  __shared__ float s_st[kDbWaves][DS::QV][2];        // per wave: running max, sum
+  __shared__ float s_m[DS::QV], s_inv[DS::QV], s_d[DS::QV];
+  __shared__ int s_odd;                              // some q or dO value is not finite
+  const int g = p.g, R = DS::QV / g;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int q4 = lane >> 4, c16 = lane & 15;
+  const int64_t per_bh = udiv32(p.n + R - 1, R);
+  const int64_t bh = udiv32(blockIdx.x, per_bh);
+  const int64_t slot0 = (blockIdx.x - bh * per_bh) * R;
+  const int64_t bb = udiv32(bh, p.h_kv);
+  const int h = static_cast<int>(bh - bb * p.h_kv);
+  float* q_lds = reinterpret_cast<float*>(db_lds);
+  float* do_lds = q_lds + DS::QV * DS::ROW;
+  unsigned char* rest = db_lds + DS::qd_bytes;
+  float* tr = reinterpret_cast<float*>(rest) + wave * DS::wave_floats;
+  KeyWindow kw;
+  kw.cnt = reinterpret_cast<uint32_t*>(rest + DS::tr_bytes);
+  kw.stride = key_window_stride(window);
+  const int cnt_words = R * kw.stride / 2, live_words = window / kKeyTile / 32 + 1;
+  kw.live = kw.cnt + cnt_words;
+  uint16_t* tiles = reinterpret_cast<uint16_t*>(kw.live + live_words) + wave * (window / kKeyTile / kDbWaves);
+
+  if (tid == 0) s_odd = 0;
+  if (tid < R) {
+    int64_t row = slot0 + tid < p.n ? slot0 + tid : -1;
+    if (row >= 0 && p.order) {
+      row = p.order[bh * p.n + slot0 + tid];
+      if (row < 0 || row >= p.n) {
+        if (p.err) p.err[0] = 1;
+        row = -1;
+      }
+    }
+    s_row[tid] = row;
+  }
+  __syncthreads();
+  {
+    // q and dO rows to LDS, D = dO . o (a wave per query vector, lane = feature)
+    bool odd = false;
+    for (int qv = wave; qv < DS::QV; qv += kDbWaves) {
+      const int r = qv / g, hh = qv - r * g;
+      const bool ok = r < R && s_row[r] >= 0;
+      const int64_t i = ok ? s_row[r] : 0;
+      const int hq = h * g + (ok ? hh : 0);
+      float od = 0.0f;
+#pragma unroll
+      for (int y = 0; y < VQ; ++y) {
+        const int dim = 64 * y + lane;
+        const float qx = ok ? static_cast<const float*>(p.q)[bb * p.q_sb + i * p.q_sn + hq * p.q_sh + dim] : 0.0f;
+        const float dx = ok ? ld_any(p.dout, bb * p.do_sb + i * p.do_sn + hq * p.do_sh + dim, p.do_bf16) : 0.0f;
+        const float ox = ok ? ld_any(p.o, bb * p.o_sb + i * p.o_sn + hq * p.o_sh + dim, p.o_bf16) : 0.0f;
+        q_lds[qv * DS::ROW + dim] = qx;
+        do_lds[qv * DS::ROW + dim] = dx;
+        odd |= !isfinite(qx) || !isfinite(dx);
+        od = fma_rn(dx, ox, od);
+      }
+      od = wave_sum(od);
+      if (lane == 0) s_d[qv] = od;
+    }
+    if (__ballot(odd) != 0ull && lane == 0) s_odd = 1;
+  }
+  const float* kbase = static_cast<const float*>(p.k) + bb * p.k_sb + static_cast<int64_t>(h) * p.k_sh;
+  const float* vbase = static_cast<const float*>(p.v) + bb * p.v_sb + static_cast<int64_t>(h) * p.v_sh;
+  int crow[QT];  // first count of the lane's query row
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) crow[qt] = min((16 * qt + c16) / g, R - 1) * kw.stride + 4 * q4;
+
+  // counts and live tiles of the window at w0; returns the wave's live tiles
+  auto fill = [&](int64_t w0) -> int {
+    kw.key0 = w0;
+    kw.len = static_cast<int>(min(static_cast<int64_t>(window), p.n - w0));
+    __syncthreads();
+    for (int e = tid; e < cnt_words + live_words; e += NTH) kw.cnt[e] = 0u;
+    __syncthreads();
+    for (int r = wave; r < R; r += kDbWaves) {
+      const int64_t row = s_row[r];
+      if (row < 0) continue;
+      const int64_t ib = bb * p.idx_sb + row * p.idx_sn + static_cast<int64_t>(h) * p.idx_sh;
+      auto load = [&](int64_t e) -> int64_t {
+        return p.idx_i64 ? static_cast<const int64_t*>(p.idx)[ib + e]
+                         : static_cast<int64_t>(static_cast<const int32_t*>(p.idx)[ib + e]);
+      };
+      strided_batches<4, 64>(p.top_k, lane, load, [&](int64_t, int64_t j) {
+        if (j < 0 || j >= p.n) {
+          if (p.err) p.err[0] = 1;
+        } else if (!(p.causal && j > row)) {
+          kw.mark(r, j);
+        }
+      });
+    }
+    __syncthreads();
+    return list_live_tiles<kDbWaves>(kw.live, static_cast<int>(ceil_div(kw.len, kKeyTile)), tiles, wave, lane);
+  };
+  // A-operand rows of a K or V tile (lane: key c16, features 16 kb + 4 q4 ..)
+  auto load_rows = [&](const float* base, int64_t sn, int64_t j0, float4 (&d)[KB]) {
+    const int64_t j = min(j0 + c16, p.n - 1);  // (past n: count 0)
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) d[kb] = *reinterpret_cast<const float4*>(base + j * sn + 16 * kb + 4 * q4);
+  };
+  // (tile rows) . (query vector rows of tile qt): lane (q4, c16) gets keys 4 q4 + e
+  auto products = [&](const float4 (&a)[KB], const float* rows, int qt) {
+    floatx4_t s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      const float4 b = *reinterpret_cast<const float4*>(rows + (16 * qt + c16) * DS::ROW + 16 * kb + 4 * q4);
+      s = __builtin_amdgcn_mfma_f32_16x16x4f32(a[kb].x, b.x, s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_16x16x4f32(a[kb].y, b.y, s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_16x16x4f32(a[kb].z, b.z, s, 0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_16x16x4f32(a[kb].w, b.w, s, 0, 0, 0);
+    }
+    return s;
+  };
+  auto counts = [&](int qt, int tile, uint32_t (&cn)[4]) {
+    const uint2 c2 =
+        *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(kw.cnt) + crow[qt] + tile * kKeyTile);
+    cn[0] = c2.x & 0xFFFFu; cn[1] = c2.x >> 16; cn[2] = c2.y & 0xFFFFu; cn[3] = c2.y >> 16;
+  };
+
+  // ---- pass 1: per query vector the max and sum over its slots (exp2 domain)
+  int nlive = 0;
+  {
+    float m_run[QT], l_run[QT];
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      m_run[qt] = -INFINITY;
+      l_run[qt] = 0.0f;
+    }
+    for (int64_t w0 = 0; w0 < p.n; w0 += window) {
+      nlive = fill(w0);
+      float4 kf[KB];
+      if (nlive > 0) load_rows(kbase, p.k_sn, w0 + static_cast<int64_t>(tiles[0]) * kKeyTile, kf);
+      for (int u = 0; u < nlive; ++u) {
+        const int tile = tiles[u];
+        floatx4_t sv[QT];
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) sv[qt] = products(kf, q_lds, qt);
+        if (u + 1 < nlive) load_rows(kbase, p.k_sn, w0 + static_cast<int64_t>(tiles[u + 1]) * kKeyTile, kf);
+#pragma unroll
+        for (int qt = 0; qt < QT; ++qt) {
+          uint32_t cn[4];
+          counts(qt, tile, cn);
+          float sc[4], mx = -INFINITY;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            sc[e] = cn[e] ? sv[qt][e] * p.qk_scale_log2 : -INFINITY;
+            mx = fmaxf(mx, sc[e]);
+          }
+          mx = rows4_reduce(mx, [](float a, float b) { return fmaxf(a, b); });
+          const float mnew = fmaxf(m_run[qt], mx);
+          const bool dead = mnew == -INFINITY;
+          float ps = 0.0f;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            ps += (dead || !cn[e]) ? 0.0f : exp2f(sc[e] - mnew) * static_cast<float>(cn[e]);
+          l_run[qt] = l_run[qt] * (dead ? 1.0f : exp2f(m_run[qt] - mnew)) + ps;
+          m_run[qt] = mnew;
+        }
+      }
+    }
+#pragma unroll
+    for (int qt = 0; qt < QT; ++qt) {
+      const float lt = rows4_reduce(l_run[qt], [](float a, float b) { return a + b; });
+      if (q4 == 0) {
+        s_st[wave][16 * qt + c16][0] = m_run[qt];
+        s_st[wave][16 * qt + c16][1] = lt;
+      }
+    }
+    __syncthreads();
+    if (tid < DS::QV) {
+      float M = -INFINITY, L = 0.0f;
+#pragma unroll
+      for (int w = 0; w < kDbWaves; ++w) M = fmaxf(M, s_st[w][tid][0]);
+#pragma unroll
+      for (int w = 0; w < kDbWaves; ++w)
+        if (s_st[w][tid][0] != -INFINITY) L += exp2f(s_st[w][tid][0] - M) * s_st[w][tid][1];
+      s_m[tid] = M == -INFINITY ? 0.0f : M;
+      s_inv[tid] = L > 0.0f ? 1.0f / L : (L == 0.0f ? 0.0f : L);  // (a NaN stays one)
+    }
+    __syncthreads();
+  }
+
+  // ---- pass 2
+  const bool odd_qd = s_odd != 0;
+  float mq[QT], iq[QT], dd[QT];
+  floatx4_t dq[QT][NT];
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt) {
+    mq[qt] = s_m[16 * qt + c16];
+    iq[qt] = s_inv[16 * qt + c16];
+    dd[qt] = s_d[16 * qt + c16];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) dq[qt][t] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  const int64_t krow = static_cast<int64_t>(p.h_kv) * D;
+  float* dkb = p.dk + (bb * p.n * p.h_kv + h) * D;
+  float* dvb = p.dv + (bb * p.n * p.h_kv + h) * D;
+  const bool one_window = p.n <= window;
+  for (int64_t w0 = 0; w0 < p.n; w0 += window) {
+    if (!one_window) nlive = fill(w0);  // else pass 1's counts and tiles stand
+    float4 kf[KB], vf[KB];
+    if (nlive > 0) {
+      load_rows(kbase, p.k_sn, w0 + static_cast<int64_t>(tiles[0]) * kKeyTile, kf);
+      load_rows(vbase, p.v_sn, w0 + static_cast<int64_t>(tiles[0]) * kKeyTile, vf);
+    }
+    for (int u = 0; u < nlive; ++u) {
+      const int tile = tiles[u];
+      const int64_t j0 = w0 + static_cast<int64_t>(tile) * kKeyTile;
+      float4 kp[4][VQ];  // K^T operand: keys 4 q4 + e, features 64 y + 4 c16 ..
+      bool odd = false;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int y = 0; y < VQ; ++y) {
+          kp[e][y] = *reinterpret_cast<const float4*>(kbase + min(j0 + 4 * q4 + e, p.n - 1) * p.k_sn + 64 * y + 4 * c16);
+          odd |= !(isfinite(kp[e][y].x) && isfinite(kp[e][y].y) && isfinite(kp[e][y].z) && isfinite(kp[e][y].w));
+        }
+      const bool slow_k = __ballot(odd) != 0ull;
+      floatx4_t dkt[NT], dvt[NT];
+#pragma unroll
+      for (int t = 0; t < NT; ++t) dkt[t] = dvt[t] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int qt = 0; qt < QT; ++qt) {
+        const floatx4_t sv = products(kf, q_lds, qt);
+        const floatx4_t dp = products(vf, do_lds, qt);
+        if (qt == QT - 1 && u + 1 < nlive) {
+          const int64_t jn = w0 + static_cast<int64_t>(tiles[u + 1]) * kKeyTile;
+          load_rows(kbase, p.k_sn, jn, kf);
+          load_rows(vbase, p.v_sn, jn, vf);
+        }
+        uint32_t cn[4];
+        counts(qt, tile, cn);
+        float pr[4], ds[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          pr[e] = cn[e] ? exp2f(sv[e] * p.qk_scale_log2 - mq[qt]) * iq[qt] * static_cast<float>(cn[e]) : 0.0f;
+          ds[e] = cn[e] ? pr[e] * (dp[e] - dd[qt]) : 0.0f;
+        }
+        // [query vector][key]
+        *reinterpret_cast<float4*>(tr + c16 * kDbTr + 4 * q4) = make_float4(pr[0], pr[1], pr[2], pr[3]);
+        *reinterpret_cast<float4*>(tr + (16 + c16) * kDbTr + 4 * q4) = make_float4(ds[0], ds[1], ds[2], ds[3]);
+        if (!slow_k) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+              const float4 k4 = kp[e][t / 4];
+              const float a = (t & 3) == 0 ? k4.x : (t & 3) == 1 ? k4.y : (t & 3) == 2 ? k4.z : k4.w;
+              dq[qt][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, ds[e], dq[qt][t], 0, 0, 0);
+            }
+        } else {
+#pragma unroll 1
+          for (int x = 0; x < kKeyTile; ++x) {
+            const int src = (x >> 2) * 16 + c16, e = x & 3;
+            const float de = __shfl(e == 0 ? ds[0] : e == 1 ? ds[1] : e == 2 ? ds[2] : ds[3], src);
+            const bool on = __shfl(static_cast<int>(e == 0 ? cn[0] : e == 1 ? cn[1] : e == 2 ? cn[2] : cn[3]), src) != 0;
+            const float* kr = kbase + min(j0 + x, p.n - 1) * p.k_sn;
+            if (on) {
+#pragma unroll
+              for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int y = 0; y < 4; ++y)
+                  dq[qt][t][y] = fma_rn(de, kr[4 * (4 * q4 + y) + (t & 3) + 64 * (t / 4)], dq[qt][t][y]);
+            }
+          }
+        }
+        wave_lds_sync();
+        if (!odd_qd) {
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {  // query vectors 4x + q4
+            const float pa = tr[(4 * x + q4) * kDbTr + c16];
+            const float da = tr[(16 + 4 * x + q4) * kDbTr + c16];
+            const float* dor = do_lds + (16 * qt + 4 * x + q4) * DS::ROW + c16;
+            const float* qr = q_lds + (16 * qt + 4 * x + q4) * DS::ROW + c16;
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+              dvt[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa, dor[16 * t], dvt[t], 0, 0, 0);
+              dkt[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(da, qr[16 * t], dkt[t], 0, 0, 0);
+            }
+          }
+        } else {
+#pragma unroll 1
+          for (int qv = 0; qv < 16; ++qv) {
+            const float* dor = do_lds + (16 * qt + qv) * DS::ROW + c16;
+            const float* qr = q_lds + (16 * qt + qv) * DS::ROW + c16;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const float pa = tr[qv * kDbTr + 4 * q4 + e], da = tr[(16 + qv) * kDbTr + 4 * q4 + e];
+              if (pa == 0.0f && da == 0.0f) continue;  // not selected, or no weight
+#pragma unroll
+              for (int t = 0; t < NT; ++t) {
+                dvt[t][e] = fma_rn(pa, dor[16 * t], dvt[t][e]);
+                dkt[t][e] = fma_rn(da, qr[16 * t], dkt[t][e]);
+              }
+            }
+          }
+        }
+        wave_lds_sync();  // tr is rewritten by the next tile
+      }
+      // dV and dK of the tile: through LDS, so that each atomic instruction adds 64
+      // consecutive floats of one key
+      auto add_tile = [&](const floatx4_t (&x)[NT], float* dst, float scale) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) tr[(4 * q4 + e) * DS::ROW + 16 * t + c16] = x[t][e] * scale;
+        wave_lds_sync();
+#pragma unroll
+        for (int key = 0; key < kKeyTile; ++key)
+#pragma unroll
+          for (int y = 0; y < VQ; ++y)
+            if (j0 + key < p.n) unsafeAtomicAdd(dst + (j0 + key) * krow + 64 * y + lane, tr[key * DS::ROW + 64 * y + lane]);
+        wave_lds_sync();
+      };
+      add_tile(dvt, dvb, 1.0f);
+      add_tile(dkt, dkb, p.inv_scale);
+    }
+  }
+
+  // ---- dQ: the waves' parts summed
+  __syncthreads();
+  float* part = reinterpret_cast<float*>(rest);
+#pragma unroll
+  for (int qt = 0; qt < QT; ++qt)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int y = 0; y < VQ; ++y)
+        *reinterpret_cast<float4*>(part + (wave * DS::QV + 16 * qt + c16) * DS::ROW + 64 * y + 4 * (4 * q4 + e)) =
+            make_float4(dq[qt][4 * y][e], dq[qt][4 * y + 1][e], dq[qt][4 * y + 2][e], dq[qt][4 * y + 3][e]);
+  __syncthreads();
+  for (int e = tid; e < R * g * (D / 4); e += NTH) {
+    const int qv = e / (D / 4), x = e - qv * (D / 4);
+    const int r = qv / g, hh = qv - r * g;
+    if (s_row[r] < 0) continue;
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int w = 0; w < kDbWaves; ++w) {
+      const float4 a = *reinterpret_cast<const float4*>(part + (w * DS::QV + qv) * DS::ROW + 4 * x);
+      o.x += a.x; o.y += a.y; o.z += a.z; o.w += a.w;
+    }
+    *reinterpret_cast<float4*>(p.dq + ((bb * p.n + s_row[r]) * p.h_q + h * g + hh) * D + 4 * x) =
+        make_float4(o.x * p.inv_scale, o.y * p.inv_scale, o.z * p.inv_scale, o.w * p.inv_scale);
+  }
+}
+
+// Taken while n <= 12 top_k (d = 64) or 5 top_k (d = 128): its time grows with n,
+// the row kernel's with top_k, both with g.  Random selections on MI355X, us, row
+// kernel / this one:
+//   d = 64   8 kv heads, g = 1:  n = 2048, k = 256: 2197 / 667;  k = 128: 1098 / 568;  k = 64: 564 / 603
+//            2 kv heads, g = 4:  n = 2048, k = 256: 990 / 497;   k = 128: 506 / 505
+//            2 kv heads, g = 8:  n = 1024, k = 128: 667 / 264;   n = 2048, k = 128: 937 / 936
+//   d = 128  2 kv heads, g = 4:  n = 2048, k = 512: 2568 / 1721; k = 256: 1293 / 1716
+//            8 kv heads, g = 1:  n = 1024, k = 128: 1157 / 520
+constexpr int kDbKeysPerSlot64 = 12, kDbKeysPerSlot128 = 5;
+constexpr int64_t kDbTwoTiles = 32 * 256;  // query vectors
+
+bool dense_bwd_f32_ok(const BwdParams& p) {
+  const auto rows16 = [](const void* x, int64_t sb, int64_t sn, int64_t sh) {
+    return reinterpret_cast<uintptr_t>(x) % 16 == 0 && sb % 4 == 0 && sn % 4 == 0 && sh % 4 == 0;
+  };
+  return (p.d == 64 || p.d == 128) && p.top_k < (1 << 16) &&
+         p.n <= static_cast<int64_t>(p.top_k) * (p.d == 64 ? kDbKeysPerSlot64 : kDbKeysPerSlot128) && rows16(p.k, p.k_sb, p.k_sn, p.k_sh) &&
+         rows16(p.v, p.v_sb, p.v_sn, p.v_sh) && reinterpret_cast<uintptr_t>(p.dq) % 16 == 0;
+}
+
+template <int D, int QT>
+int launch_dense_bwd_f32(const BwdParams& p, hipStream_t st) {
+  using DS = DbShape<D, QT>;
+  const int R = DS::QV / p.g;
+  const int window = key_window(p.n, R, kDbCountBytes);
+  const size_t lds = DS::lds(R, window);
+  if (int s = reserve_lds(reinterpret_cast<const void*>(dense_bwd_f32_kernel<D, QT>), lds, "dense_bwd_f32_kernel"))
+    return s;
+  const int64_t blocks = (p.rows / p.n) * ceil_div(p.n, R);
+  dense_bwd_f32_kernel<D, QT><<<dim3(static_cast<unsigned>(blocks)), 64 * kDbWaves, lds, st>>>(p, window);
+  return check_launch("dense_bwd_f32_kernel");
+}
+
 template <typename T, int GMAX>
 int launch_bwd_g(const BwdParams& p, hipStream_t st) {
   const dim3 grid(static_cast<unsigned>(ceil_div(p.rows, kBwdWaves)));
@@ -1568,6 +1996,14 @@ int launch_bwd(const BwdParams& p, hipStream_t st) {
         prefix_attention_bwd_kernel<128, false><<<pgrid, 64 * w, 0, st>>>(p);
       }
       return check_launch("prefix_attention_bwd_kernel");
+    }
+  }
+  if constexpr (sizeof(T) == 4) {
+    if (dense_bwd_f32_ok(p)) {
+      const int64_t qvs = p.rows * p.g;
+      if (p.d == 64)
+        return qvs >= kDbTwoTiles ? launch_dense_bwd_f32<64, 2>(p, st) : launch_dense_bwd_f32<64, 1>(p, st);
+      return launch_dense_bwd_f32<128, 1>(p, st);
     }
   }
   if (p.g <= 4) return launch_bwd_g<T, 4>(p, st);

@@ -84,3 +84,63 @@ def test_dense_f32_flags_and_order(dev):
     assert int(flag.item()) == 1 and (part[0, 9] == 7.0).all()
     keep = torch.arange(n) != 9
     assert torch.equal(part[0, keep], good[0, keep])
+
+
+def _backward_oracle(orc, q, kk, v, idx, dout, causal):
+    return orc.sparse_attention_backward(f32(q[0]), f32(kk[0]), f32(v[0]), idx[0].to(torch.int64).numpy(),
+                                         dout[0].double().numpy(), causal=causal)
+
+
+@pytest.mark.parametrize("d,g,h_kv,n,k,causal,i64", [
+    (64, 1, 2, 1999, 300, False, True),    # several key windows, counted again for the second pass
+    (64, 3, 2, 331, 70, True, False),      # 15 of 16 query vectors used
+    (64, 4, 4, 700, 130, True, True),      # two query tiles a block
+    (128, 5, 1, 257, 100, True, True),
+    (128, 16, 1, 40, 40, False, False),
+    (64, 8, 1, 17, 30, False, True)])      # k > n: padded with key 0
+def test_dense_f32_backward_vs_oracle(dev, orc, d, g, h_kv, n, k, causal, i64):
+    from ssa_amd import kernels
+
+    q, kk, v, idx = _case(n, h_kv, g, d, min(k, n), 51)
+    dout = randn((1, n, h_kv * g, d), 55)
+    if k > n:
+        idx = torch.cat((idx, idx.new_zeros(1, n, h_kv, k - n)), dim=-1)
+    elif k < n:
+        idx[..., 1] = idx[..., 0]
+    idx = idx if i64 else idx.to(torch.int32)
+    order = torch.stack([torch.randperm(n) for _ in range(h_kv)]).to(torch.int32)[None].to(dev)
+    args = [t.to(dev) for t in (q, kk, v, idx)]
+    out = kernels.sparse_attention(*args, None, causal)
+    flag = torch.zeros(1, dtype=torch.int32, device=dev)
+    got = kernels.sparse_attention_backward(*args, out, dout.to(dev), None, causal, error_flag=flag, row_order=order)
+    assert int(flag.item()) == 0
+    for x, ref in zip(got, _backward_oracle(orc, q, kk, v, idx, dout, causal)):
+        # as tests/test_gpu_backward.py: 32-bit sums, atomics in any order
+        assert np.abs(x[0].cpu().numpy() - ref).max() <= 2e-5 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("what", ["k", "dout"])
+def test_dense_f32_backward_keeps_non_finite_values_apart(dev, orc, what):
+    """A key's or an output gradient's infinity reaches what its own pairs feed, nothing else."""
+    from ssa_amd import kernels
+
+    n, h_kv, g, d, k, at = 80, 1, 4, 64, 24, 11
+    q, kk, v, idx = _case(n, h_kv, g, d, k, 61)
+    dout = randn((1, n, g, d), 65)
+    args = [t.to(dev) for t in (q, kk, v, idx)]
+    out = kernels.sparse_attention(*args)
+    has = torch.zeros(n, n, dtype=torch.bool).scatter_(1, idx[0, :, 0], True)   # row selects key
+    ref = _backward_oracle(orc, q, kk, v, idx, dout, False)
+    if what == "k":
+        args[1][0, at, 0, 3] = float("inf")
+        rows, keys = has[:, at], None
+    else:
+        dout[0, at, 2, 5] = float("inf")
+        rows, keys = torch.arange(n) == at, has[at]
+    if keys is None:
+        keys = has[rows].any(0)
+    got = [x[0].cpu() for x in kernels.sparse_attention_backward(*args, out, dout.to(dev))]
+    for x, r, touched in ((got[0], ref[0], rows), (got[1], ref[1], keys), (got[2], ref[2], keys)):
+        if bool((~touched).any()):
+            np.testing.assert_allclose(x[~touched].numpy(), r[(~touched).numpy()], rtol=0, atol=2e-5 * np.abs(r).max())
+    assert not got[0][rows].isfinite().all() and not got[1][keys].isfinite().all()
