@@ -207,6 +207,160 @@ size_t route_vectors_tile_smem(int d) {
   return sizeof(float) * (static_cast<size_t>(32 + kRvRows) * (d + 4) + static_cast<size_t>(kRvRows) * 32);
 }
 
+// head_dim 64 or 128, route_dim <= 32 and a multiple of 4: the projections on the
+// fp32 matrix cores.  v_mfma_f32_32x32x2_f32 computes each product sum as fmaf
+// chains in ascending order (checked bit for bit against fmaf, denormals
+// included), so a chain of d / 2 of them over W (rows: the 32 coordinates) and x
+// (columns: 32 tokens) is the canonical chain of every (token, coordinate).
+//   block   four waves, 128 tokens of one (batch, output head); a wave runs its
+//           32 tokens' heads one after the other and folds them in head order;
+//   W       in LDS once per block, split into even and odd dimensions, so that
+//           lane (half, row) reads four steps' operands (dimensions 2s + half) at
+//           once;
+//   x       a lane loads LB consecutive bytes of its token's row (lanes 0-31 the
+//           first half of a piece of 2 LB bytes, lanes 32-63 the second), the next
+//           piece while this one is multiplied; v_permlane32_swap then gives both
+//           lanes of a token both halves;
+//   result  lane (half, token) holds coordinates 8j + 4 half .. + 3; the norm's
+//           chain needs them in order, again through v_permlane32_swap.
+// Queries and keys go in one launch (the second tensor's blocks after the first's).
+// The vector-ALU kernels below keep other head dims and unaligned rows.
+// Bound by the row loads' latency beside the MFMA chains (68 us at the fp32 matrix
+// rate): queries and keys of n = 32768, 32/8 heads, d = 128, bf16 take 131 us, on
+// the vector ALUs 222 us in two launches (63% of their rate); the fp32 README
+// layer (batch 2, n = 1024, 8/2 heads, d = 64) 13 us against 56 us.
+struct RouteIn {
+  const void* x;
+  int64_t n;
+  int h_in, group;
+  int64_t sb, sn, sh;
+  const float* w;
+  float* out;
+};
+constexpr int kRmRows = 128;  // tokens per block
+
+// {the lower 32 lanes' value, the upper 32 lanes' value} of x, in every lane
+struct HalfPair {
+  uint32_t lo, hi;
+};
+__device__ __forceinline__ HalfPair both_halves(uint32_t x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  return HalfPair{r[0], r[1]};
+}
+
+template <typename T, int DC>
+__global__ __launch_bounds__(256, 4) void route_vectors_mfma_kernel(RouteIn a, RouteIn b, int64_t blocks_a, int d_s) {
+  typedef float floatx16_t __attribute__((ext_vector_type(16)));
+  constexpr int ROWB = DC * static_cast<int>(sizeof(T));
+  constexpr int LB = ROWB / 2 < 128 ? ROWB / 2 : 128;  // bytes a lane loads per piece
+  constexpr int NL = LB / 16, NCH = ROWB / (2 * LB);
+  constexpr int SPH = LB / static_cast<int>(sizeof(T)) / 2;  // MFMA steps per half piece
+  constexpr int WS = DC / 2 + 4;                              // floats per W row and half
+  __shared__ __align__(16) float wl[2][32][WS];
+  const bool second = blockIdx.x >= blocks_a;
+  const RouteIn p = second ? b : a;
+  const int64_t blk = second ? blockIdx.x - blocks_a : blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5, c = lane & 31;
+  const int h_out = p.h_in / p.group;
+  const int64_t tiles = udiv32(p.n + kRmRows - 1, kRmRows);
+  const int64_t bh = udiv32(blk, tiles);
+  const int64_t i = (blk - bh * tiles) * kRmRows + 32 * wave + c;
+  const int64_t bb = udiv32(bh, h_out);
+  const int h = static_cast<int>(bh - bb * h_out);
+  const T* xr = static_cast<const T*>(p.x) + bb * p.sb + static_cast<int64_t>(h) * p.group * p.sh +
+                min(i, p.n - 1) * p.sn;  // tokens past n: the last one, not stored
+  for (int e = tid; e < 32 * (DC / 4); e += 256) {
+    const int s = e / (DC / 4), t4 = e - s * (DC / 4);
+    const float4 w4 = s < d_s ? *reinterpret_cast<const float4*>(p.w + s * DC + 4 * t4) : make_float4(0.f, 0.f, 0.f, 0.f);
+    *reinterpret_cast<float2*>(&wl[0][s][2 * t4]) = make_float2(w4.x, w4.z);
+    *reinterpret_cast<float2*>(&wl[1][s][2 * t4]) = make_float2(w4.y, w4.w);
+  }
+  auto load = [&](int gg, int ch, uint4 (&d)[NL]) {
+    const uint4* src = reinterpret_cast<const uint4*>(
+        reinterpret_cast<const char*>(xr + static_cast<int64_t>(gg) * p.sh) + ch * 2 * LB + half * LB);
+#pragma unroll
+    for (int l = 0; l < NL; ++l) d[l] = src[l];
+  };
+  uint4 cur[NL], nxt[NL];
+  load(0, 0, cur);
+  __syncthreads();
+  const uint32_t sel = half ? 0x03020C0Cu : 0x01000C0Cu;  // bf16 pair -> this half's value as fp32
+  float sum[16];
+  int w0 = (32 * half + c) * WS;  // the lane's W row
+  for (int gg = 0; gg < p.group; ++gg) {
+    asm volatile("" : "+v"(w0));  // read again for each head: kept in registers W costs a wave per SIMD
+    const float* wr = &wl[0][0][0] + w0;
+    floatx16_t acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+#pragma unroll
+    for (int ch = 0; ch < NCH; ++ch) {
+      if (ch + 1 < NCH) load(gg, ch + 1, nxt);
+      else if (gg + 1 < p.group) load(gg + 1, 0, nxt);
+#pragma unroll
+      for (int side = 0; side < 2; ++side) {
+        const int s0 = (2 * ch + side) * SPH;  // first step
+#pragma unroll
+        for (int l = 0; l < NL; ++l) {
+          const uint32_t u[4] = {cur[l].x, cur[l].y, cur[l].z, cur[l].w};
+          uint32_t v[4];
+#pragma unroll
+          for (int y = 0; y < 4; ++y) {
+            const HalfPair hp = both_halves(u[y]);
+            v[y] = side ? hp.hi : hp.lo;
+          }
+          if constexpr (sizeof(T) == 2) {
+            const float4 w4 = *reinterpret_cast<const float4*>(wr + s0 + 4 * l);
+            const float wv[4] = {w4.x, w4.y, w4.z, w4.w};
+#pragma unroll
+            for (int y = 0; y < 4; ++y)
+              acc = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[y], __uint_as_float(__builtin_amdgcn_perm(0u, v[y], sel)),
+                                                         acc, 0, 0, 0);
+          } else {
+            const float2 w2 = *reinterpret_cast<const float2*>(wr + s0 + 2 * l);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(w2.x, __uint_as_float(half ? v[1] : v[0]), acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(w2.y, __uint_as_float(half ? v[3] : v[2]), acc, 0, 0, 0);
+          }
+        }
+      }
+#pragma unroll
+      for (int l = 0; l < NL; ++l) cur[l] = nxt[l];
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) sum[r] = gg == 0 ? acc[r] : sum[r] + acc[r];
+  }
+  float lo[16], hi[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    sum[r] = sum[r] / static_cast<float>(p.group);
+    const HalfPair hp = both_halves(__float_as_uint(sum[r]));
+    lo[r] = __uint_as_float(hp.lo);
+    hi[r] = __uint_as_float(hp.hi);
+  }
+  float nrm = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {  // coordinates 4j .. 4j + 3
+    if (4 * j < d_s) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float v = (j & 1) ? hi[4 * (j / 2) + e] : lo[4 * (j / 2) + e];
+        nrm = fma_rn(v, v, nrm);
+      }
+    }
+  }
+  const float den = fmaxf(sqrtf(nrm), 1e-12f);
+  if (i < p.n) {
+    float* o = p.out + (bh * p.n + i) * d_s + 4 * half;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (8 * j + 4 * half < d_s)
+        *reinterpret_cast<float4*>(o + 8 * j) =
+            make_float4(sum[4 * j] / den, sum[4 * j + 1] / den, sum[4 * j + 2] / den, sum[4 * j + 3] / den);
+  }
+}
+
 // route_dim == 32, head_dim a multiple of 8: one lane per output row, all 32
 // coordinates in registers.  W is the same for every lane, so its
 // entries are wave-uniform scalar loads (s_load) and every fmaf takes its W
@@ -236,12 +390,11 @@ __device__ __forceinline__ Piece8 load8(const float* p) {
   return Piece8{{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}};
 }
 
-template <typename T, int DC>
+template <typename T>
 __global__ __launch_bounds__(kRrThreads) void route_vectors_row_kernel(
-    const T* __restrict__ x, int64_t n, int h_in, int group, int d_rt, int64_t sb, int64_t sn,
+    const T* __restrict__ x, int64_t n, int h_in, int group, int d, int64_t sb, int64_t sn,
     int64_t sh, const float* __restrict__ w, float* __restrict__ out) {
   constexpr int d_s = 32;
-  const int d = DC > 0 ? DC : d_rt;
   const int h_out = h_in / group;
   const int64_t tiles = (n + kRrThreads - 1) / kRrThreads;
   const int64_t bh = udiv32(blockIdx.x, tiles);
@@ -256,37 +409,28 @@ __global__ __launch_bounds__(kRrThreads) void route_vectors_row_kernel(
   float sum[32], acc[32];
 #pragma unroll
   for (int s = 0; s < 32; ++s) sum[s] = acc[s] = 0.0f;
-  // With d fixed at compile time, 8 pieces per unrolled step: every W
-  // operand of the step is an immediate offset from one base, so the scalar
-  // loads of several pieces go out together (one piece per step waits on its
-  // W loads every dozen fmas).
-  constexpr int UNR = DC > 0 && DC % 64 == 0 ? 8 : 1;
   Piece8 cur = load8(xb);
 #pragma unroll 1
-  for (int c0 = 0; c0 < total; c0 += UNR) {
+  for (int c = 0; c < total; ++c) {
+    const int gg = c / pieces;
+    const int t0 = (c - gg * pieces) * 8;
+    const int cn = c + 1 < total ? c + 1 : c;
+    const int ggn = cn / pieces;
+    const Piece8 nxt = load8(xb + static_cast<int64_t>(ggn) * sh + (cn - ggn * pieces) * 8);
 #pragma unroll
-    for (int u = 0; u < UNR; ++u) {
-      const int c = c0 + u;
-      const int gg = c / pieces;
-      const int t0 = (c - gg * pieces) * 8;
-      const int cn = c + 1 < total ? c + 1 : c;
-      const int ggn = cn / pieces;
-      const Piece8 nxt = load8(xb + static_cast<int64_t>(ggn) * sh + (cn - ggn * pieces) * 8);
+    for (int s = 0; s < d_s; ++s) {
+      const float* ws = w + static_cast<int64_t>(s) * d + t0;
 #pragma unroll
-      for (int s = 0; s < d_s; ++s) {
-        const float* ws = w + static_cast<int64_t>(s) * d + t0;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[s] = fma_rn(cur.v[e], ws[e], acc[s]);
-      }
-      if (t0 + 8 == d) {  // head gg complete: fold its chain into the group sum
-#pragma unroll
-        for (int s = 0; s < 32; ++s) {
-          sum[s] = (gg == 0) ? acc[s] : sum[s] + acc[s];
-          acc[s] = 0.0f;
-        }
-      }
-      cur = nxt;
+      for (int e = 0; e < 8; ++e) acc[s] = fma_rn(cur.v[e], ws[e], acc[s]);
     }
+    if (t0 + 8 == d) {  // head gg complete: fold its chain into the group sum
+#pragma unroll
+      for (int s = 0; s < 32; ++s) {
+        sum[s] = (gg == 0) ? acc[s] : sum[s] + acc[s];
+        acc[s] = 0.0f;
+      }
+    }
+    cur = nxt;
   }
   float nrm = 0.0f;
 #pragma unroll
@@ -299,76 +443,6 @@ __global__ __launch_bounds__(kRrThreads) void route_vectors_row_kernel(
     float* o = out + (bh * n + i) * d_s;
 #pragma unroll
     for (int s = 0; s < d_s; ++s) o[s] = sum[s] / den;
-  }
-}
-
-// One head per output row (group == 1, the keys), route_dim == 32, bf16 rows of
-// a fixed head dim: route_vectors_row_kernel with each row's 32 coordinates
-// split over two waves of a block (wave 0: coordinates 0-15, wave 1: 16-31,
-// the same 64 rows), so twice the waves share the same fmaf chains and each
-// wave's W rows are still wave-uniform scalar loads.  The norm chain runs over
-// the coordinates in order: wave 0 passes its partial sum of squares to wave 1
-// through LDS, wave 1 finishes it and passes the denominator back.  Same
-// results as route_vectors_row_kernel, bit for bit.
-constexpr int kRhRows = 64;
-template <int DC>
-__global__ __launch_bounds__(128) void route_vectors_half_kernel(
-    const uint16_t* __restrict__ x, int64_t n, int h_in, int64_t sb, int64_t sn, int64_t sh,
-    const float* __restrict__ w, float* __restrict__ out) {
-  constexpr int HS = 16;  // coordinates per wave
-  constexpr int pieces = DC / 8;
-  constexpr int UNR = pieces % 8 == 0 ? 8 : 1;
-  __shared__ float s_nrm[kRhRows], s_den[kRhRows];
-  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const int lane = threadIdx.x & 63;
-  const int64_t tiles = (n + kRhRows - 1) / kRhRows;
-  const int64_t bh = udiv32(blockIdx.x, tiles);
-  const int64_t i = (blockIdx.x - bh * tiles) * kRhRows + lane;
-  const int64_t b = udiv32(bh, h_in);
-  const int h = static_cast<int>(bh - b * h_in);
-  const int64_t ic = i < n ? i : n - 1;  // lanes past n compute row n-1 and store nothing
-  const uint16_t* xr = x + b * sb + static_cast<int64_t>(h) * sh + ic * sn;
-  const float* wh = w + static_cast<int64_t>(wave * HS) * DC;
-  float acc[HS];
-#pragma unroll
-  for (int s = 0; s < HS; ++s) acc[s] = 0.0f;
-  Piece8 cur = load8(xr);
-#pragma unroll 1
-  for (int c0 = 0; c0 < pieces; c0 += UNR) {
-#pragma unroll
-    for (int u = 0; u < UNR; ++u) {
-      const int c = c0 + u;
-      const int cn = c + 1 < pieces ? c + 1 : c;
-      const Piece8 nxt = load8(xr + cn * 8);
-#pragma unroll
-      for (int s = 0; s < HS; ++s) {
-        const float* ws = wh + s * DC + c * 8;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[s] = fma_rn(cur.v[e], ws[e], acc[s]);
-      }
-      cur = nxt;
-    }
-  }
-  // (the group mean divides by 1: unchanged)
-  float nrm = 0.0f;
-  if (wave == 0) {
-#pragma unroll
-    for (int s = 0; s < HS; ++s) nrm = fma_rn(acc[s], acc[s], nrm);
-    s_nrm[lane] = nrm;
-  }
-  __syncthreads();
-  if (wave == 1) {
-    nrm = s_nrm[lane];
-#pragma unroll
-    for (int s = 0; s < HS; ++s) nrm = fma_rn(acc[s], acc[s], nrm);
-    s_den[lane] = fmaxf(sqrtf(nrm), 1e-12f);
-  }
-  __syncthreads();
-  const float den = s_den[lane];
-  if (i < n) {
-    float* o = out + (bh * n + i) * 32 + wave * HS;
-#pragma unroll
-    for (int s = 0; s < HS; ++s) o[s] = acc[s] / den;
   }
 }
 
@@ -415,12 +489,11 @@ __device__ __forceinline__ Piece8 line_piece(const Line128& l, int pi) {
   return r;
 }
 
-template <typename T, int DC>
+template <typename T>
 __global__ __launch_bounds__(256) void route_vectors_split_kernel(
-    const T* __restrict__ x, int64_t n, int h_in, int group, int d_rt, int64_t sb, int64_t sn,
+    const T* __restrict__ x, int64_t n, int h_in, int group, int d, int64_t sb, int64_t sn,
     int64_t sh, const float* __restrict__ w, float* __restrict__ out) {
   constexpr int d_s = 32;
-  const int d = DC > 0 ? DC : d_rt;
   __shared__ float part[4][kRsRows][d_s + 1];  // per-wave head chains, padded rows
   __shared__ float mean[kRsRows][d_s + 1];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -1399,6 +1472,31 @@ int check_route_vectors(int dtype, int64_t batch, int64_t n, int h_in, int group
   return SSA_OK;
 }
 
+// The matrix-core projection of one tensor, or of queries and keys in one launch
+// (b.x null: a alone).
+bool route_mfma_ok(int dtype, const RouteIn& r, int d, int d_s) {
+  const int64_t pe = dtype == SSA_DTYPE_BF16 ? 8 : 4;  // elements per 16 bytes
+  return (d == 64 || d == 128) && d_s <= 32 && d_s % 4 == 0 && r.sb % pe == 0 && r.sn % pe == 0 && r.sh % pe == 0 &&
+         reinterpret_cast<uintptr_t>(r.x) % 16 == 0 && reinterpret_cast<uintptr_t>(r.w) % 16 == 0 &&
+         reinterpret_cast<uintptr_t>(r.out) % 16 == 0;
+}
+
+int launch_route_mfma(const RouteIn& a, const RouteIn& b, int dtype, int64_t batch, int d, int d_s, hipStream_t st) {
+  const auto blocks = [&](const RouteIn& r) {
+    return r.x ? batch * (r.h_in / r.group) * ceil_div(r.n, kRmRows) : 0;
+  };
+  const int64_t na = blocks(a), nb = blocks(b);
+  const dim3 grid(static_cast<unsigned>(na + nb));
+  if (dtype == SSA_DTYPE_BF16) {
+    if (d == 64) route_vectors_mfma_kernel<uint16_t, 64><<<grid, 256, 0, st>>>(a, b, na, d_s);
+    else route_vectors_mfma_kernel<uint16_t, 128><<<grid, 256, 0, st>>>(a, b, na, d_s);
+  } else {
+    if (d == 64) route_vectors_mfma_kernel<float, 64><<<grid, 256, 0, st>>>(a, b, na, d_s);
+    else route_vectors_mfma_kernel<float, 128><<<grid, 256, 0, st>>>(a, b, na, d_s);
+  }
+  return check_launch("route_vectors_mfma_kernel");
+}
+
 int launch_route_vectors(const void* x, int dtype, int64_t batch, int64_t n, int h_in, int group,
                          int d, int64_t sb, int64_t sn, int64_t sh, const float* w, int d_s,
                          float* out, hipStream_t st) {
@@ -1417,33 +1515,25 @@ int launch_route_vectors(const void* x, int dtype, int64_t batch, int64_t n, int
     FewRoute none{};
     return launch_route_few(t0, none, dtype, st);
   }
+  const RouteIn in{x, n, h_in, group, sb, sn, sh, w, out};
+  if (route_mfma_ok(dtype, in, d, d_s)) return launch_route_mfma(in, RouteIn{}, dtype, batch, d, d_s, st);
   if (d_s == 32 && piece8 && group > 1) {
     const int64_t grid = batch * (h_in / group) * ceil_div(n, kRsRows);
     if (dtype == SSA_DTYPE_BF16)
-      if (d == 128)
-        route_vectors_split_kernel<uint16_t, 128><<<dim3(static_cast<unsigned>(grid)), 256, 0, st>>>(
-            static_cast<const uint16_t*>(x), n, h_in, group, d, sb, sn, sh, w, out);
-      else
-        route_vectors_split_kernel<uint16_t, 0><<<dim3(static_cast<unsigned>(grid)), 256, 0, st>>>(
-            static_cast<const uint16_t*>(x), n, h_in, group, d, sb, sn, sh, w, out);
+      route_vectors_split_kernel<uint16_t><<<dim3(static_cast<unsigned>(grid)), 256, 0, st>>>(
+          static_cast<const uint16_t*>(x), n, h_in, group, d, sb, sn, sh, w, out);
     else
-      route_vectors_split_kernel<float, 0><<<dim3(static_cast<unsigned>(grid)), 256, 0, st>>>(
+      route_vectors_split_kernel<float><<<dim3(static_cast<unsigned>(grid)), 256, 0, st>>>(
           static_cast<const float*>(x), n, h_in, group, d, sb, sn, sh, w, out);
     return check_launch("route_vectors_split_kernel");
-  }
-  if (d_s == 32 && piece8 && group == 1 && dtype == SSA_DTYPE_BF16 && d == 128) {
-    const int64_t grid = batch * h_in * ceil_div(n, kRhRows);
-    route_vectors_half_kernel<128><<<dim3(static_cast<unsigned>(grid)), 128, 0, st>>>(
-        static_cast<const uint16_t*>(x), n, h_in, sb, sn, sh, w, out);
-    return check_launch("route_vectors_half_kernel");
   }
   if (d_s == 32 && piece8) {
     const int64_t grid = batch * (h_in / group) * ceil_div(n, kRrThreads);
     if (dtype == SSA_DTYPE_BF16)
-      route_vectors_row_kernel<uint16_t, 0><<<dim3(static_cast<unsigned>(grid)), kRrThreads, 0, st>>>(
+      route_vectors_row_kernel<uint16_t><<<dim3(static_cast<unsigned>(grid)), kRrThreads, 0, st>>>(
           static_cast<const uint16_t*>(x), n, h_in, group, d, sb, sn, sh, w, out);
     else
-      route_vectors_row_kernel<float, 0><<<dim3(static_cast<unsigned>(grid)), kRrThreads, 0, st>>>(
+      route_vectors_row_kernel<float><<<dim3(static_cast<unsigned>(grid)), kRrThreads, 0, st>>>(
           static_cast<const float*>(x), n, h_in, group, d, sb, sn, sh, w, out);
     return check_launch("route_vectors_row_kernel");
   }
@@ -2157,10 +2247,15 @@ extern "C" int ssa_route_codes(const void* q, const void* k, int dtype, int64_t 
   float* chat = reinterpret_cast<float*>(static_cast<char*>(workspace) + 2 * vec);
   void* tws = static_cast<char*>(workspace) + 2 * vec +
               align_up(sizeof(float) * static_cast<size_t>(h_kv) * n_c * d_s, 256);
-  if ((st = launch_route_vectors(q, dtype, batch, n, h_q, g, d, q_sb, q_sn, q_sh, w_qr, d_s, qhat, s)))
-    return st;
-  if ((st = launch_route_vectors(k, dtype, batch, n, h_kv, 1, d, k_sb, k_sn, k_sh, w_kr, d_s, khat, s)))
-    return st;
+  const RouteIn rq{q, n, h_q, g, q_sb, q_sn, q_sh, w_qr, qhat}, rk{k, n, h_kv, 1, k_sb, k_sn, k_sh, w_kr, khat};
+  if (batch * h_kv * n > kLaneRowsMax && route_mfma_ok(dtype, rq, d, d_s) && route_mfma_ok(dtype, rk, d, d_s)) {
+    if ((st = launch_route_mfma(rq, rk, dtype, batch, d, d_s, s))) return st;
+  } else {
+    if ((st = launch_route_vectors(q, dtype, batch, n, h_q, g, d, q_sb, q_sn, q_sh, w_qr, d_s, qhat, s)))
+      return st;
+    if ((st = launch_route_vectors(k, dtype, batch, n, h_kv, 1, d, k_sb, k_sn, k_sh, w_kr, d_s, khat, s)))
+      return st;
+  }
   if ((st = launch_normalize(codebook, static_cast<int64_t>(h_kv) * n_c, d_s, chat, s))) return st;
   // top 16 for the queries and top 4 for the keys (config 3's a and b): both
   // screens in one launch, the keys' flag bytes after the workspace's others
