@@ -20,6 +20,7 @@
 //              this order (their set is every candidate), so only rows with
 //              more than k candidates are rescored.
 #include <mutex>
+#include <type_traits>
 
 #include "ssa_common.h"
 #include "ssa_internal.h"
@@ -588,6 +589,186 @@ __device__ __forceinline__ void sort_slots_desc(uint64_t* keys, int lane) {
   for (int r = 0; r < E; ++r) keys[lane * E + r] = x[r];
 }
 
+
+// ---- exact scores of 64 keys on the matrix cores --------------------------------
+//
+// v_mfma_f32_4x4x1_16b_f32 takes one dimension of 16 independent 4 x 4 products:
+// lane l's own key as column l % 4 of block l / 4 and the group's query head l % 4 as
+// row, so each lane ends with its key's dot products with four heads, and a chain of
+// D of them over ascending dimensions is the canonical fmaf chain, bit for bit
+// (checked against fmaf, denormals included).  That is half the issue time of the
+// vector ALU's chains and leaves it to the bf16 conversions.
+// qs: the query rows in LDS as fp32, row stride kQsRow (rows past g zero).
+template <int D>
+constexpr int kQsRow = D + 4;  // rows start 4 banks apart
+
+// 64 dimensions t0 .. of the lane's bf16 key (kv: eight pieces of eight).
+template <int GI, int D>
+__device__ __forceinline__ void exact_step64(const uint4 (&kv)[8], const float* qs, int t0, int lane,
+                                             floatx4_t (&acc)[GI]) {
+#pragma unroll
+  for (int gi = 0; gi < GI; ++gi) {
+    const float* qr = qs + (4 * gi + (lane & 3)) * kQsRow<D> + t0;
+#pragma unroll
+    for (int x = 0; x < 16; ++x) {
+      const float4 q = *reinterpret_cast<const float4*>(qr + 4 * x);
+      const uint32_t w0 = (x & 1) ? kv[x / 2].z : kv[x / 2].x, w1 = (x & 1) ? kv[x / 2].w : kv[x / 2].y;
+      acc[gi] = __builtin_amdgcn_mfma_f32_4x4x1f32(q.x, __uint_as_float(w0 << 16), acc[gi], 0, 0, 0);
+      acc[gi] = __builtin_amdgcn_mfma_f32_4x4x1f32(q.y, __uint_as_float(w0 & 0xFFFF0000u), acc[gi], 0, 0, 0);
+      acc[gi] = __builtin_amdgcn_mfma_f32_4x4x1f32(q.z, __uint_as_float(w1 << 16), acc[gi], 0, 0, 0);
+      acc[gi] = __builtin_amdgcn_mfma_f32_4x4x1f32(q.w, __uint_as_float(w1 & 0xFFFF0000u), acc[gi], 0, 0, 0);
+    }
+  }
+}
+
+// Query rows of the group to LDS for exact_step64 (threads 0 .. NT - 1).
+template <int GMAX, int D, int NT>
+__device__ __forceinline__ void stage_queries(const uint16_t* q0, int64_t q_sh, int g, float* qs, int tid) {
+  for (int x = tid; x < GMAX * (D / 8); x += NT) {
+    const int gg = x / (D / 8), t = (x % (D / 8)) * 8;
+    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (gg < g) load8(q0 + static_cast<int64_t>(gg) * q_sh + t, v);
+    *reinterpret_cast<float4*>(qs + gg * kQsRow<D> + t) = make_float4(v[0], v[1], v[2], v[3]);
+    *reinterpret_cast<float4*>(qs + gg * kQsRow<D> + t + 4) = make_float4(v[4], v[5], v[6], v[7]);
+  }
+}
+
+// The row's score from the per-head dot products: mean over heads of dot / score_div.
+template <int GI>
+__device__ __forceinline__ float score_of_acc(const SelParams& p, const floatx4_t (&acc)[GI]) {
+  float sc = acc[0][0] / p.score_div;
+#pragma unroll
+  for (int gg = 1; gg < 4 * GI; ++gg)
+    if (gg < p.g) sc = sc + acc[gg / 4][gg % 4] / p.score_div;
+  return sc / static_cast<float>(p.g);
+}
+
+// select_sort_kernel for bf16 rows of 64 or 128 features: the key rows of 64 slots
+// at a time go to LDS by buffer loads, 128 bytes of each row per step, so that a
+// load instruction moves eight whole cache lines (a lane reading its own row in
+// 16-byte pieces touches 64 of them per instruction).  A step's rows go on to
+// registers at once and the one buffer takes the next step's while they are
+// multiplied: 10 KB of LDS a wave, 15 waves a CU.  Segments are XOR-swizzled by row / 2, so the
+// lanes' reads of their own rows hit distinct banks.
+// n = 32768, 32/8 heads, d = 128, k = 512: 1.78 ms against 2.88 ms with the
+// vector-ALU chains of select_sort_kernel on rows read lane by lane (81% of the time
+// in address processing); n = 131072, 16/2 heads, k = 1024: 12.8 against 14.3 ms.
+// With two buffers (18 KB a wave, half the waves) it gained 4% only: the gathers
+// want waves in flight.
+template <int GMAX, int D>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(GMAX <= 4 ? 4 : 3, 8))) void
+select_sort_rows_kernel(SelParams p, const uint16_t* __restrict__ qg) {
+  constexpr int GI = GMAX / 4, NH = D / 64;  // 64-feature steps per chunk of 64 keys
+  constexpr int EM = kSortMax / 64;
+  __shared__ __align__(16) unsigned char kbuf[64 * 128];
+  __shared__ __align__(16) float qs[GMAX * kQsRow<D>];
+  const int lane = threadIdx.x;
+  const int64_t row = row_of_slot(p, blockIdx.x);
+  if (row < 0) return;
+  const int m = min(p.cnt[row], p.k_eff);
+  if (m <= 1) return;
+  const int64_t bh = udiv32(row, p.n_q);
+  const int64_t r = row - bh * p.n_q;
+  const int64_t bb = udiv32(bh, p.h_kv);
+  const int h = static_cast<int>(bh - bb * p.h_kv);
+  const uint16_t* q0 = qg + bb * p.q_sb + r * p.q_sn + static_cast<int64_t>(h * p.g) * p.q_sh;
+  const uint16_t* kbase = static_cast<const uint16_t*>(p.k) + bb * p.k_sb + static_cast<int64_t>(h) * p.k_sh;
+  const int64_t obase = ((bb * p.n_q + r) * p.h_kv + h) * p.top_k;
+  int32_t* o32 = static_cast<int32_t*>(p.out) + obase;
+  int64_t* o64 = static_cast<int64_t*>(p.out) + obase;
+  stage_queries<GMAX, D, 64>(q0, p.q_sh, p.g, qs, lane);
+
+  // key of slot 64 c + lane in x[c] (its low word until the score is known)
+  uint64_t x[EM];
+  const int nch = (m + 63) >> 6;
+  // (low words of int32 or int64 entries; slots past m read entry m - 1, a row that
+  // exists, so that no branch waits between the loads)
+  const int ewords = p.out_i64 ? 2 : 1;
+  const uint32_t* owords = p.out_i64 ? reinterpret_cast<const uint32_t*>(o64) : reinterpret_cast<const uint32_t*>(o32);
+#pragma unroll
+  for (int c = 0; c < EM; ++c) x[c] = owords[min(64 * c + lane, m - 1) * ewords];
+  const uint32_t ksn2 = 2u * static_cast<uint32_t>(p.k_sn);
+  const int kbytes = static_cast<int>((p.n - 1) * p.k_sn * 2 + 2 * D);
+  const __amdgpu_buffer_rsrc_t krs =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(kbase), 0, kbytes, kBufferWord3);
+  auto key_of = [&](int c) -> int32_t {
+    uint32_t j = 0;
+#pragma unroll
+    for (int e = 0; e < EM; ++e) j = e == c ? static_cast<uint32_t>(x[e]) : j;
+    return static_cast<int32_t>(j);
+  };
+  // Load t moves 128 bytes of rows 8t .. 8t + 7: lane l the segment that belongs in
+  // slot l % 8 of row 8t + l / 8.
+  uint32_t off[8];
+  auto set_rows = [&](int c) {
+    const int32_t j = key_of(c);
+#pragma unroll
+    for (int t = 0; t < 8; ++t) {
+      const int rr = 8 * t + (lane >> 3);
+      off[t] = __umul24(static_cast<uint32_t>(__shfl(j, rr)), ksn2) +
+               static_cast<uint32_t>(((lane & 7) ^ ((rr >> 1) & 7)) << 4);
+    }
+  };
+  auto issue = [&](int hf) {
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(krs, (lds_void_ptr)(kbuf + t * 1024), 16,
+                                               static_cast<int>(off[t] + 128u * hf), 0, 0, 0);
+  };
+  wave_lds_sync();
+  set_rows(0);
+  issue(0);
+#pragma unroll 1
+  for (int c = 0; c < nch; ++c) {
+    floatx4_t acc[GI];
+#pragma unroll
+    for (int gi = 0; gi < GI; ++gi) acc[gi] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int hf = 0; hf < NH; ++hf) {
+      __builtin_amdgcn_s_waitcnt(kWaitVm0);
+      asm volatile("" ::: "memory");
+      const unsigned char* kr = kbuf + lane * 128;
+      uint4 kv[8];
+#pragma unroll
+      for (int t = 0; t < 8; ++t) kv[t] = *reinterpret_cast<const uint4*>(kr + ((t ^ ((lane >> 1) & 7)) << 4));
+      // the rows are in registers: the buffer takes the next step's
+      __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+      asm volatile("" ::: "memory");
+      if (hf + 1 < NH) {
+        issue(hf + 1);
+      } else if (c + 1 < nch) {
+        set_rows(c + 1);
+        issue(0);
+      }
+      exact_step64<GI, D>(kv, qs, 64 * hf, lane, acc);
+    }
+    const float sc = score_of_acc<GI>(p, acc);
+    const uint64_t key = 64 * c + lane < m ? composite_key(sc, static_cast<uint32_t>(key_of(c))) : 0ull;
+#pragma unroll
+    for (int e = 0; e < EM; ++e) x[e] = e == c ? key : x[e];
+  }
+  auto sorted_out = [&](auto e_c) {
+    constexpr int E = decltype(e_c)::value;
+    uint64_t y[E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) y[e] = x[e];
+    wave_sort_desc<E>(y, lane);
+#pragma unroll
+    for (int e = 0; e < E; ++e) {  // slot lane E + e
+      const int slot = lane * E + e;
+      const int32_t j = static_cast<int32_t>(key_index(y[e]));
+      if (slot < m) {
+        if (p.out_i64) o64[slot] = j;
+        else o32[slot] = j;
+      }
+    }
+  };
+  if (nch <= 1) sorted_out(std::integral_constant<int, 1>{});
+  else if (nch <= 2) sorted_out(std::integral_constant<int, 2>{});
+  else if (nch <= 4) sorted_out(std::integral_constant<int, 4>{});
+  else if (nch <= 8) sorted_out(std::integral_constant<int, 8>{});
+  else sorted_out(std::integral_constant<int, 16>{});
+}
 
 template <typename T, int GMAX, int D>
 __global__ __launch_bounds__(64) void select_sort_kernel(SelParams p, const T* __restrict__ qg) {
@@ -1856,6 +2037,12 @@ int launch_select(const SelParams& p, int64_t rows, size_t smem, void* ws, size_
   hk<<<dim3(static_cast<unsigned>(persistent_grid(rows, 8))), kSelThreads, smem, st>>>(pi, qg, w);
   if (int s = check_launch("select_heavy_kernel")) return s;
   if (!sort_after) return SSA_OK;
+  if constexpr (kScreenable) {
+    if (screen) {
+      select_sort_rows_kernel<GMAX, D><<<dim3(static_cast<unsigned>(rows)), 64, 0, st>>>(pi, qg);
+      return check_launch("select_sort_rows_kernel");
+    }
+  }
   select_sort_kernel<T, GMAX, D><<<dim3(static_cast<unsigned>(rows)), 64, 0, st>>>(pi, qg);
   return check_launch("select_sort_kernel");
 }
