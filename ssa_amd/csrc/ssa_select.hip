@@ -19,6 +19,7 @@
 //              filler.  Rows with at most k candidates need no scores at all in
 //              this order (their set is every candidate), so only rows with
 //              more than k candidates are rescored.
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -152,6 +153,7 @@ __device__ void bitonic_desc(uint64_t* buf, int len) {
 }
 
 // Exclusive block-wide prefix sum of v; *total receives the block sum.
+template <int NT = kSelThreads>
 __device__ int block_exclusive_scan(int v, int* scratch, int* total) {
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -160,7 +162,7 @@ __device__ int block_exclusive_scan(int v, int* scratch, int* total) {
   __syncthreads();
   int base = 0, tot = 0;
 #pragma unroll
-  for (int w = 0; w < kSelThreads / 64; ++w) {
+  for (int w = 0; w < NT / 64; ++w) {
     const int s = scratch[w];
     if (w < wave) base += s;
     tot += s;
@@ -173,11 +175,12 @@ __device__ int block_exclusive_scan(int v, int* scratch, int* total) {
 // Writes, in ascending order, the first `limit` positions j < n whose bitmap bit
 // equals `want_set` to dst[0..]; returns how many were written.  Only words
 // below `live` are stored; the rest read as zero.
+template <int NT = kSelThreads>
 __device__ int scan_bits(const uint32_t* bitmap, int words, int live, int64_t n, bool want_set,
                          int32_t* dst, int limit, int* scratch) {
   int filled = 0;
   const int wend = want_set ? live : words;
-  for (int w0 = 0; w0 < wend && filled < limit; w0 += kSelThreads) {
+  for (int w0 = 0; w0 < wend && filled < limit; w0 += NT) {
     const int w = w0 + threadIdx.x;
     uint32_t bits = 0u;
     if (w < wend) {
@@ -186,7 +189,7 @@ __device__ int scan_bits(const uint32_t* bitmap, int words, int live, int64_t n,
       if (w == words - 1 && (n & 31)) bits &= (1u << (n & 31)) - 1u;
     }
     int total = 0;
-    int rank = filled + block_exclusive_scan(__popc(bits), scratch, &total);
+    int rank = filled + block_exclusive_scan<NT>(__popc(bits), scratch, &total);
     while (bits != 0u && rank < limit) {
       const int bpos = __ffs(bits) - 1;
       bits &= bits - 1u;
@@ -853,6 +856,206 @@ template <typename T, int GMAX, int D>
 __global__ __launch_bounds__(kSelThreads) void select_kernel(SelParams p, const T* __restrict__ qg) {
   const int64_t row = row_of_slot(p, blockIdx.x);
   if (row >= 0) select_row<T, GMAX, D>(p, qg, row, false);
+}
+
+// A few rows in index order (decoding): one block of 1024 threads per row, so that
+// every step of a row runs in one or two rounds of memory latency.  A call of eight
+// rows leaves the rest of the GPU idle, and select_row's 256 threads went through
+// the postings, the candidates and their key rows in several rounds each:
+//   union    one posting per thread; a key whose bitmap bit was clear joins the
+//            candidate list;
+//   scores   (more than k_eff candidates) one candidate per thread, bf16 rows of 64
+//            or 128 features as exact matrix chains (exact_step64);
+//   cut      the k_eff-th largest composite key by 8-bit digits (a barrier per digit;
+//            a bitonic sort of 1024 keys takes 55); smaller keys leave the bitmap;
+//   output   the bitmap's keys ascending, then the filler.
+// A row with more than kFewCap candidates goes on as select_row, on the first 256
+// threads (the other waves end).  Same results.
+// Eight rows over a cache of 32700 keys (32/8 heads, 16 codes, k = 512): 15 us against
+// 45 us; the decoding step 79 -> 51 us.
+constexpr int kFewThreads = 1024;
+constexpr int kFewCap = 2048;
+constexpr int64_t kFewRows = 256;  // one block per CU
+
+inline size_t select_few_smem(const SelParams& p) {
+  return sizeof(int32_t) * (8 * 256 + kFewCap + p.k_eff) +
+         sizeof(uint32_t) * static_cast<size_t>((p.n + 31) / 32);
+}
+
+template <typename T, int GMAX, int D>
+__global__ __launch_bounds__(kFewThreads) void select_few_kernel(SelParams p, const T* __restrict__ qg) {
+  constexpr bool kMatrix = sizeof(T) == 2 && (D == 64 || D == 128);
+  constexpr int GI = GMAX / 4;
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ __align__(16) float qs[kMatrix ? GMAX * kQsRow<D> : 4];
+  __shared__ int s_lo[kMaxA], s_start[kMaxA + 1];
+  __shared__ int s_cnt;
+  __shared__ int s_scan[kFewThreads / 64];
+  const int64_t row = row_of_slot(p, blockIdx.x);
+  if (row < 0) return;
+  int* hist = reinterpret_cast<int*>(smem);  // [8][256]
+  int32_t* list = reinterpret_cast<int32_t*>(hist + 8 * 256);
+  int32_t* stage = list + kFewCap;
+  uint32_t* bitmap = reinterpret_cast<uint32_t*>(stage + p.k_eff);
+  const int words = static_cast<int>((p.n + 31) >> 5);
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int64_t bh = udiv32(row, p.n_q);
+  const int64_t r = row - bh * p.n_q;
+  const int64_t i = p.q_pos0 + r;
+  const int64_t bb = udiv32(bh, p.h_kv);
+  const int h = static_cast<int>(bh - bb * p.h_kv);
+  const T* q0 = qg + bb * p.q_sb + r * p.q_sn + static_cast<int64_t>(h * p.g) * p.q_sh;
+  const T* kbase = static_cast<const T*>(p.k) + bb * p.k_sb + static_cast<int64_t>(h) * p.k_sh;
+  const int32_t* pp = p.postings + bh * p.post_bh;
+  const int32_t* tp = p.tail_postings ? p.tail_postings + bh * p.tail_bh : nullptr;
+  const bool causal = p.mask_mode == SSA_MASK_CAUSAL;
+  const uint8_t* mrow = (p.mask_mode == SSA_MASK_DENSE) ? p.mask + bb * p.mask_sb + i * p.mask_si : nullptr;
+  const int live = causal ? static_cast<int>(i >> 5) + 1 : words;
+  if (tid < 64) {  // buckets, as in select_row
+    int32_t lo = 0, len = 0;
+    if (tid < p.nseg) {
+      const bool tl = tid >= p.a;
+      const int32_t c = p.q_codes[(bh * p.n_q + r) * p.a + (tl ? tid - p.a : tid)];
+      if (static_cast<uint32_t>(c) < static_cast<uint32_t>(p.n_c)) {
+        const int32_t* off = (tl ? p.tail_offsets : p.offsets) + bh * (p.n_c + 1);
+        const int32_t total = static_cast<int32_t>(tl ? p.tail_bh : p.post_bh);
+        lo = min(max(off[c], 0), total);
+        len = min(max(off[c + 1], lo), total) - lo;
+      }
+    }
+    const int32_t x = wave_incl_scan(len);
+    if (tid < p.nseg) {
+      s_lo[tid] = lo;
+      s_start[tid + 1] = x;
+    }
+    if (tid == 0) {
+      s_start[0] = 0;
+      s_cnt = 0;
+    }
+  }
+  for (int w = tid; w < live; w += kFewThreads) bitmap[w] = 0u;
+  for (int w = tid; w < 8 * 256; w += kFewThreads) hist[w] = 0;
+  if constexpr (kMatrix) stage_queries<GMAX, D, kFewThreads>(q0, p.q_sh, p.g, qs, tid);
+  __syncthreads();
+  const int R = s_start[p.nseg];
+  for (int base = 0; base < R; base += kFewThreads) {
+    const int pidx = base + tid;
+    bool fresh = false;
+    int32_t j = 0;
+    if (pidx < R) {
+      int lo_m = 0, hi_m = p.nseg;
+      while (hi_m - lo_m > 1) {
+        const int mid = (lo_m + hi_m) >> 1;
+        if (s_start[mid] <= pidx) lo_m = mid;
+        else hi_m = mid;
+      }
+      const int32_t e = s_lo[lo_m] + (pidx - s_start[lo_m]);
+      j = lo_m < p.a ? pp[e] : tp[e] + p.tail_key0;
+      if (static_cast<uint32_t>(j) < static_cast<uint32_t>(p.n) && (!causal || j <= i) &&
+          (mrow == nullptr || mrow[j] != 0)) {
+        const uint32_t bit = 1u << (j & 31);
+        fresh = !(atomicOr(&bitmap[j >> 5], bit) & bit);
+      }
+    }
+    const uint64_t m = __ballot(fresh);
+    int at = 0;
+    if (lane == 0 && m != 0ull) at = atomicAdd(&s_cnt, __popcll(m));
+    at = lane_value(at, 0) + __popcll(m & ((1ull << lane) - 1));
+    if (fresh && at < kFewCap) list[at] = j;
+  }
+  __syncthreads();
+  const int C = s_cnt;
+  if (C > kFewCap) {
+    if (tid >= kSelThreads) return;
+    __syncthreads();
+    select_row<T, GMAX, D>(p, qg, row, false);
+    return;
+  }
+  if (C > p.k_eff) {
+    uint64_t key[kFewCap / kFewThreads];  // candidates tid, tid + 1024; 0 past C
+#pragma unroll
+    for (int x = 0; x < kFewCap / kFewThreads; ++x) {
+      const int e = x * kFewThreads + tid;
+      key[x] = 0ull;
+      if (x * kFewThreads >= C) continue;  // uniform
+      const int32_t j = list[min(e, C - 1)];
+      const T* kr = kbase + static_cast<int64_t>(j) * p.k_sn;
+      float sc;
+      if constexpr (kMatrix) {
+        floatx4_t acc[GI];
+#pragma unroll
+        for (int gi = 0; gi < GI; ++gi) acc[gi] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (int hf = 0; hf < D / 64; ++hf) {
+          uint4 kv[8];
+#pragma unroll
+          for (int t = 0; t < 8; ++t) kv[t] = reinterpret_cast<const uint4*>(kr)[8 * hf + t];
+          exact_step64<GI, D>(kv, qs, 64 * hf, lane, acc);
+        }
+        sc = score_of_acc<GI>(p, acc);
+      } else {
+        float acc[GMAX];
+        rescore_row<T, GMAX, D>(kr, q0, p.q_sh, p.g, p.d, acc);
+        sc = acc[0] / p.score_div;
+#pragma unroll
+        for (int gg = 1; gg < GMAX; ++gg)
+          if (gg < p.g) sc = sc + acc[gg] / p.score_div;
+        sc = sc / static_cast<float>(p.g);
+      }
+      if (e < C) key[x] = composite_key(sc, static_cast<uint32_t>(j));
+    }
+    // The k_eff-th largest key by 8-bit digits from the top (keys are distinct): a
+    // histogram of the keys that share the digits found so far, which every wave
+    // walks for itself; done as soon as a whole bin is selected.
+    uint64_t found = 0ull, mask = 0ull;
+    int need = p.k_eff;
+    for (int pass = 0; pass < 8; ++pass) {
+      const int shift = 56 - 8 * pass;
+#pragma unroll
+      for (int x = 0; x < kFewCap / kFewThreads; ++x)
+        if (key[x] != 0ull && (key[x] & mask) == found) atomicAdd(&hist[pass * 256 + ((key[x] >> shift) & 255)], 1);
+      __syncthreads();
+      const int* hb = hist + pass * 256 + 252 - 4 * lane;  // lane's bins, the highest first: hb[3] .. hb[0]
+      const int c3 = hb[3], c2 = hb[2], c1 = hb[1], c0 = hb[0];
+      const int incl = wave_incl_scan(c3 + c2 + c1 + c0);
+      const int src = __builtin_ctzll(__ballot(incl >= need));
+      int above = lane_value(incl - (c3 + c2 + c1 + c0), src);  // keys in higher bins
+      const int cc[4] = {lane_value(c3, src), lane_value(c2, src), lane_value(c1, src), lane_value(c0, src)};
+      int bin = 255 - 4 * src, in = cc[0];
+#pragma unroll
+      for (int y = 1; y < 4; ++y)
+        if (above + in < need) {
+          above += in;
+          in = cc[y];
+          --bin;
+        }
+      need -= above;
+      found |= static_cast<uint64_t>(bin) << shift;
+      mask |= 255ull << shift;
+      if (in == need) break;
+    }
+#pragma unroll
+    for (int x = 0; x < kFewCap / kFewThreads; ++x)
+      if (key[x] != 0ull && (key[x] & mask) < found) {
+        const uint32_t j = key_index(key[x]);
+        atomicAnd(&bitmap[j >> 5], ~(1u << (j & 31)));
+      }
+    __syncthreads();
+  }
+  const int nsel = min(C, p.k_eff);
+  scan_bits<kFewThreads>(bitmap, words, live, p.n, true, stage, nsel, s_scan);
+  __syncthreads();
+  if (nsel < p.k_eff)
+    scan_bits<kFewThreads>(bitmap, words, live, p.n, false, stage + nsel, p.k_eff - nsel, s_scan);
+  __syncthreads();
+  const int64_t obase = ((bb * p.n_q + r) * p.h_kv + h) * p.top_k;
+  for (int w = tid; w < p.top_k; w += kFewThreads) {
+    const int32_t j = w < p.k_eff ? stage[w] : 0;
+    if (p.out_i64) static_cast<int64_t*>(p.out)[obase + w] = j;
+    else static_cast<int32_t*>(p.out)[obase + w] = j;
+  }
+  if (p.prefix && tid == 0)
+    p.prefix[row] = (nsel < p.k_eff && p.k_eff == p.top_k) ? stage[p.k_eff - 1] + 1 : 0;
 }
 
 // Workspace of index order (carve_sel_ws).  Rows with more than k candidates
@@ -1984,6 +2187,15 @@ int launch_select(const SelParams& p, int64_t rows, size_t smem, void* ws, size_
   const bool screen = kScreenable && p.n < (int64_t(1) << 24) && 2 * p.k_sn < (int64_t(1) << 24) &&
                       (p.n - 1) * p.k_sn * 2 + 2 * p.d < (int64_t(1) << 31);
   if (ws == nullptr || (p.sorted && p.k_eff > kSortMax) || light_smem(p) > 64 * 1024) {
+    if (!p.sorted && !p.stats && rows <= kFewRows) {
+      const size_t fsmem = std::max(smem, select_few_smem(p));
+      auto few = select_few_kernel<T, GMAX, D>;
+      if (fsmem + sizeof(float) * GMAX * (D + 4) + 4096 <= kLdsBytesPerCu) {
+        if (int s = reserve_lds(reinterpret_cast<const void*>(few), fsmem, "select")) return s;
+        few<<<dim3(static_cast<unsigned>(rows)), kFewThreads, fsmem, st>>>(p, qg);
+        return check_launch("select_few_kernel");
+      }
+    }
     kern<<<dim3(static_cast<unsigned>(rows)), kSelThreads, smem, st>>>(p, qg);
     return check_launch("select_kernel");
   }
