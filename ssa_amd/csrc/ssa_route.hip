@@ -1277,14 +1277,75 @@ __global__ __launch_bounds__(256, 1) void code_topk_mfma_pair_kernel(
                              bh * tiles + i - tiles);
 }
 
-// Exact top-`top` codes of the rows flagged by the matrix-core filter
-// (flags[bh * rows + row] != 0), one wave per row: lane l scores codes l, l + 64,
-// ... in the canonical fp32 order (one fmaf chain over d_s, then / temperature)
-// and keeps its best TM composite keys in a sorted register list; `top` rounds
-// of a wave-wide maximum then take the row's keys in descending order.  The
-// result is the top-`top` by (score desc, code asc), as code_topk_kernel gives.
-// Each wave scans the flags of 64 consecutive rows per step, so unflagged rows
-// cost one byte read.
+// Exact top-`top` codes of one row by one wave: lane l scores codes l, l + 64, ...
+// in the canonical fp32 order (one fmaf chain over d_s, then / temperature) and
+// keeps its best TM composite keys in a sorted register list; `top` rounds of a
+// wave-wide maximum then take the row's keys in descending order.  The result is
+// the top-`top` by (score desc, code asc), as code_topk_kernel gives.
+// C codes of a lane are in flight at a time.
+template <int TM, int C>
+__device__ __forceinline__ void exact_row_topk(const float* __restrict__ xr, const float* __restrict__ cb, int n_c,
+                                               int d_s, float temperature, int top, int32_t* __restrict__ out) {
+  const int lane = threadIdx.x & 63;
+  const bool scale = (temperature != 1.0f);
+  float x[32];
+#pragma unroll
+  for (int s = 0; s < 32; ++s) x[s] = (s < d_s) ? xr[s] : 0.0f;
+  uint64_t best[TM];
+#pragma unroll
+  for (int p = 0; p < TM; ++p) best[p] = 0ull;  // below every key
+  auto insert = [&](uint64_t key) {
+#pragma unroll
+    for (int p = TM - 1; p > 0; --p) best[p] = key > best[p - 1] ? best[p - 1] : (key > best[p] ? key : best[p]);
+    best[0] = key > best[0] ? key : best[0];
+  };
+  auto load = [&](int c, float4 (&cv)[8]) {
+    const float4* cr = reinterpret_cast<const float4*>(cb + static_cast<int64_t>(c) * d_s);
+#pragma unroll
+    for (int s4 = 0; s4 < 8; ++s4) cv[s4] = (s4 * 4 < d_s) ? cr[s4] : make_float4(0.f, 0.f, 0.f, 0.f);
+  };
+  auto key_of = [&](int c, const float4 (&cv)[8]) -> uint64_t {
+    float acc = 0.0f;
+#pragma unroll
+    for (int s4 = 0; s4 < 8; ++s4) {
+      if (s4 * 4 < d_s) {
+        acc = fma_rn(x[s4 * 4 + 0], cv[s4].x, acc);
+        acc = fma_rn(x[s4 * 4 + 1], cv[s4].y, acc);
+        acc = fma_rn(x[s4 * 4 + 2], cv[s4].z, acc);
+        acc = fma_rn(x[s4 * 4 + 3], cv[s4].w, acc);
+      }
+    }
+    if (scale) acc = acc / temperature;
+    return composite_key(acc, static_cast<uint32_t>(c));
+  };
+  for (int c = lane; c < n_c; c += 64 * C) {
+    float4 cv[C][8];
+#pragma unroll
+    for (int y = 0; y < C; ++y) load(c + 64 * y < n_c ? c + 64 * y : c, cv[y]);
+#pragma unroll
+    for (int y = 0; y < C; ++y)
+      if (c + 64 * y < n_c) insert(key_of(c + 64 * y, cv[y]));
+  }
+  for (int p = 0; p < top; ++p) {
+    uint64_t v = best[0];
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const uint32_t lo = static_cast<uint32_t>(__shfl_xor(static_cast<int>(v & 0xFFFFFFFFull), o));
+      const uint32_t hi = static_cast<uint32_t>(__shfl_xor(static_cast<int>(v >> 32), o));
+      const uint64_t w = (static_cast<uint64_t>(hi) << 32) | lo;
+      v = w > v ? w : v;
+    }
+    const bool win = best[0] == v;  // keys are distinct, so one lane holds v
+#pragma unroll
+    for (int q = 0; q < TM - 1; ++q) best[q] = win ? best[q + 1] : best[q];
+    best[TM - 1] = win ? 0ull : best[TM - 1];
+    if (lane == 0) out[p] = static_cast<int32_t>(key_index(v));
+  }
+}
+
+// The rows flagged by the matrix-core filter (flags[bh * rows + row] != 0), one wave
+// per row.  Each wave scans the flags of 64 consecutive rows per step, so unflagged
+// rows cost one byte read.
 template <int TM>
 __global__ __launch_bounds__(256) void code_topk_rows_kernel(const float* __restrict__ xhat, int64_t total,
                                                              int64_t rows, int h, const float* __restrict__ chat,
@@ -1294,69 +1355,13 @@ __global__ __launch_bounds__(256) void code_topk_rows_kernel(const float* __rest
   const int lane = threadIdx.x & 63;
   const int64_t gw = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   const int64_t nw = static_cast<int64_t>(gridDim.x) * 4;
-  const bool scale = (temperature != 1.0f);
   for (int64_t base = gw * 64; base < total; base += nw * 64) {
     const bool f = base + lane < total && flags[base + lane] != 0;
     for (uint64_t m = __ballot(f); m != 0ull; m &= m - 1ull) {
       const int64_t grow = base + (__ffsll(static_cast<long long>(m)) - 1);  // bh * rows + row
       const int hh = static_cast<int>((grow / rows) % h);
-      const float* xr = xhat + grow * d_s;
-      const float* cb = chat + static_cast<int64_t>(hh) * n_c * d_s;
-      float x[32];
-#pragma unroll
-      for (int s = 0; s < 32; ++s) x[s] = (s < d_s) ? xr[s] : 0.0f;
-      uint64_t best[TM];
-#pragma unroll
-      for (int p = 0; p < TM; ++p) best[p] = 0ull;  // below every key
-      auto insert = [&](uint64_t key) {
-#pragma unroll
-        for (int p = TM - 1; p > 0; --p) best[p] = key > best[p - 1] ? best[p - 1] : (key > best[p] ? key : best[p]);
-        best[0] = key > best[0] ? key : best[0];
-      };
-      auto load = [&](int c, float4 (&cv)[8]) {
-        const float4* cr = reinterpret_cast<const float4*>(cb + static_cast<int64_t>(c) * d_s);
-#pragma unroll
-        for (int s4 = 0; s4 < 8; ++s4) cv[s4] = (s4 * 4 < d_s) ? cr[s4] : make_float4(0.f, 0.f, 0.f, 0.f);
-      };
-      auto key_of = [&](int c, const float4 (&cv)[8]) -> uint64_t {
-        float acc = 0.0f;
-#pragma unroll
-        for (int s4 = 0; s4 < 8; ++s4) {
-          if (s4 * 4 < d_s) {
-            acc = fma_rn(x[s4 * 4 + 0], cv[s4].x, acc);
-            acc = fma_rn(x[s4 * 4 + 1], cv[s4].y, acc);
-            acc = fma_rn(x[s4 * 4 + 2], cv[s4].z, acc);
-            acc = fma_rn(x[s4 * 4 + 3], cv[s4].w, acc);
-          }
-        }
-        if (scale) acc = acc / temperature;
-        return composite_key(acc, static_cast<uint32_t>(c));
-      };
-      // two codes per step, both code rows in flight before either is scored
-      for (int c = lane; c < n_c; c += 128) {
-        const bool two = c + 64 < n_c;
-        float4 cv0[8], cv1[8];
-        load(c, cv0);
-        load(two ? c + 64 : c, cv1);
-        insert(key_of(c, cv0));
-        if (two) insert(key_of(c + 64, cv1));
-      }
-      int32_t* out = codes + grow * top;
-      for (int p = 0; p < top; ++p) {
-        uint64_t v = best[0];
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-          const uint32_t lo = static_cast<uint32_t>(__shfl_xor(static_cast<int>(v & 0xFFFFFFFFull), o));
-          const uint32_t hi = static_cast<uint32_t>(__shfl_xor(static_cast<int>(v >> 32), o));
-          const uint64_t w = (static_cast<uint64_t>(hi) << 32) | lo;
-          v = w > v ? w : v;
-        }
-        const bool win = best[0] == v;  // keys are distinct, so one lane holds v
-#pragma unroll
-        for (int q = 0; q < TM - 1; ++q) best[q] = win ? best[q + 1] : best[q];
-        best[TM - 1] = win ? 0ull : best[TM - 1];
-        if (lane == 0) out[p] = static_cast<int32_t>(key_index(v));
-      }
+      exact_row_topk<TM, 2>(xhat + grow * d_s, chat + static_cast<int64_t>(hh) * n_c * d_s, n_c, d_s, temperature, top,
+                            codes + grow * top);
     }
   }
 }
@@ -1592,6 +1597,236 @@ struct FewTopk {
   int top;
   int32_t* codes;     // [total][top]
 };
+
+// Candidates a row of code_topk_tile_kernel may hold.
+constexpr int kTileCap = 112;
+
+// Top codes of a moderate number of rows, queries and keys in one launch: one block
+// per 16 NT rows of a (batch, head), its four waves splitting the codebook, the same
+// screen and bound as code_topk_mfma_block otherwise.
+//   pass 1   wave w takes tiles 8w .. 8w + 7, 8w + 32 .., keeping M segment maxima per
+//            lane and row; a row's 16 M maxima of the block's 16 lanes go through LDS,
+//            where its 256 / (16 NT) lanes count, for each, the maxima above it: the
+//            least with fewer than `top` above is the top-th largest;
+//   pass 2   hits go to the row's list in LDS, in any order;
+//   pass 3   the row's lanes rescore its list exactly, one code each at a time, and a
+//            code's place is the number of keys above its own (keys are distinct).
+// Rows whose list overflows (or whose bound is not finite) run exhaustively here, one
+// wave each.  With 256 rows a block, such a call left most CUs idle and a wave went
+// through the whole codebook twice for its 64 rows, one lane through a row's list:
+// bound by that chain (README layer, 4096 rows, N_c 2048: 84 us; route_codes 107 -> 40 us;
+// 406 rows, N_c 512: 75 -> 36 us).
+template <int NT, int TM>
+__global__ __launch_bounds__(256) void code_topk_tile_kernel(FewTopk ta, FewTopk tb, int h,
+                                                             const float* __restrict__ chat,
+                                                             const uint16_t* __restrict__ cbf,
+                                                             const uint32_t* __restrict__ cmax_bits, int n_c, int d_s,
+                                                             float temperature, int64_t tiles, int64_t nblocks) {
+  constexpr int R = 16 * NT, L = 256 / R;          // rows of the block, lanes per row
+  constexpr int M = (NT == 1 || TM > 16) ? 4 : 2;  // segment maxima per lane and row
+  constexpr int S = 16 * M, SR = S + 1;
+  constexpr int KR = kTileCap + 1;
+  static_assert(sizeof(float) * SR <= sizeof(uint64_t) * KR, "the maxima fit the lists");
+  __shared__ uint64_t keys[R * KR];  // a row's candidates: codes, then their keys
+  __shared__ float s_lb[R];
+  __shared__ int s_cnt[R], s_bad[R];
+  float* segs = reinterpret_cast<float*>(keys);  // [R][SR], before pass 2
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int q4 = lane >> 4, c16 = lane & 15;
+
+  const int64_t lb = xcd_block(blockIdx.x, xcd_per(nblocks));
+  if (lb >= nblocks) return;
+  const int64_t per = (tb.total > 0 ? 2 : 1) * tiles;  // blocks per (batch, head): queries', then keys'
+  const int64_t bh = udiv32(lb, per), i = lb - bh * per;
+  const FewTopk& t = i < tiles ? ta : tb;
+  const int top = t.top;
+  const int64_t r0 = (i < tiles ? i : i - tiles) * R;
+  const int hh = static_cast<int>(bh - udiv32(bh, h) * h);
+  const int n_c_pad = n_c_padded(n_c), ntile = n_c_pad / 16;
+  const float* xb = t.xhat + bh * t.rows * d_s;
+  const uint16_t* cbh = cbf + static_cast<int64_t>(hh) * n_c_pad * 32;
+  const float* cb = chat + static_cast<int64_t>(hh) * n_c * d_s;
+  auto row4 = [&](int64_t row, int s4) -> float4 {
+    return (row < t.rows && 4 * s4 < d_s) ? *reinterpret_cast<const float4*>(xb + row * d_s + 4 * s4)
+                                          : make_float4(0.f, 0.f, 0.f, 0.f);
+  };
+  // tiles tt .. tt + 7 of the bf16 codebook (tiles past the end repeat the last one)
+  auto load8 = [&](bf16x8_t (&a)[8], int tt) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      a[u] = *reinterpret_cast<const bf16x8_t*>(cbh + (static_cast<int64_t>(min(tt + u, ntile - 1)) * 16 + c16) * 32 +
+                                                q4 * 8);
+  };
+
+  bf16x8_t a[8];
+  load8(a, 8 * wave);
+  bf16x8_t bfrag[NT];
+  float eps[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const int64_t row = r0 + nt * 16 + c16;
+    const float4 x0 = row4(row, 2 * q4), x1 = row4(row, 2 * q4 + 1);
+    const float f[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+    uint16_t tmp[8];
+    float nrm2 = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      tmp[e] = bf16_rne(f[e]);
+      nrm2 = fma_rn(f[e], f[e], nrm2);
+    }
+    bfrag[nt] = __builtin_bit_cast(bf16x8_t, tmp);
+    nrm2 += __shfl_xor(nrm2, 16);
+    nrm2 += __shfl_xor(nrm2, 32);
+    eps[nt] = kMfEps * sqrtf(nrm2) * __uint_as_float(cmax_bits[hh]) * 1.0001f;
+    if (wave == 0 && q4 == 0) {
+      s_bad[nt * 16 + c16] = !(eps[nt] <= 3.0e38f);
+      s_cnt[nt * 16 + c16] = 0;
+    }
+  }
+
+  // ---- pass 1
+  float smax[NT][M];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int u = 0; u < M; ++u) smax[nt][u] = -INFINITY;
+  for (int tt = 8 * wave; tt < ntile; tt += 32) {
+    bf16x8_t an[8];
+    load8(an, tt + 32);
+    const bool edge = (tt + 8) * 16 > n_c;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        floatx4_t sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], bfrag[nt], floatx4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        if (edge) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if ((tt + u) * 16 + q4 * 4 + e >= n_c) sc[e] = -INFINITY;
+        }
+        float& m = smax[nt][u % M];
+        m = vmax(vmax(vmax(sc[0], sc[1]), sc[2]), vmax(sc[3], m));
+      }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a[u] = an[u];
+  }
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int u = 0; u < M; ++u) segs[(nt * 16 + c16) * SR + (wave * 4 + q4) * M + u] = smax[nt][u];
+  load8(a, 8 * wave);
+  __syncthreads();
+  const int r = tid / L, sub = tid % L;
+  {
+    constexpr int V = S / L;
+    float v[V];
+    int above[V];
+#pragma unroll
+    for (int x = 0; x < V; ++x) {
+      v[x] = segs[r * SR + x * L + sub];
+      above[x] = 0;
+    }
+#pragma unroll 8
+    for (int j = 0; j < S; ++j) {
+      const float o = segs[r * SR + j];
+#pragma unroll
+      for (int x = 0; x < V; ++x) above[x] += o > v[x] ? 1 : 0;
+    }
+    float lbv = INFINITY;
+#pragma unroll
+    for (int x = 0; x < V; ++x)
+      if (above[x] < top) lbv = fminf(lbv, v[x]);
+#pragma unroll
+    for (int o = 1; o < L; o <<= 1) lbv = fminf(lbv, __shfl_xor(lbv, o));
+    if (sub == 0) s_lb[r] = lbv;
+  }
+  __syncthreads();  // (and the maxima are read: pass 2 writes over them)
+
+  // ---- pass 2 (the scores minus the threshold, their signs gathered per 8 tiles, as
+  // code_topk_mfma_block has it)
+  floatx4_t cneg[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    float thr = s_lb[nt * 16 + c16] - 2.0f * eps[nt];
+    if (r0 + nt * 16 + c16 >= t.rows || !(eps[nt] <= 3.0e38f) || !(thr == thr)) thr = INFINITY;
+    cneg[nt] = floatx4_t{-thr, -thr, -thr, -thr};
+  }
+  for (int tt = 8 * wave; tt < ntile; tt += 32) {
+    bf16x8_t an[8];
+    load8(an, tt + 32);
+    uint32_t bits[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) bits[nt] = 0u;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) {
+        const floatx4_t d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], bfrag[nt], cneg[nt], 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bits[nt] = __builtin_amdgcn_alignbit(bits[nt], __float_as_uint(d[e]), 31);
+      }
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+      uint32_t hm = ~bits[nt];
+      while (hm) {
+        const int b = __builtin_ctz(hm);
+        hm &= hm - 1u;
+        const int v = 31 - b;  // 4u + e
+        const int code = tt * 16 + ((v >> 2) << 4) + 4 * q4 + (v & 3);
+        if (code < n_c) {
+          const int at = atomicAdd(&s_cnt[nt * 16 + c16], 1);
+          if (at < kTileCap) keys[(nt * 16 + c16) * KR + at] = static_cast<uint64_t>(code);
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a[u] = an[u];
+  }
+  __syncthreads();
+
+  // ---- pass 3
+  const int m = s_cnt[r];
+  const bool over = s_bad[r] != 0 || m > kTileCap || m < top;
+  const bool mine = r0 + r < t.rows && !over;
+  uint64_t* kr = keys + r * KR;
+  if (mine) {
+    float4 xr[8];
+#pragma unroll
+    for (int s4 = 0; s4 < 8; ++s4) xr[s4] = row4(r0 + r, s4);
+    for (int e = sub; e < m; e += L) {
+      const int c = static_cast<int>(kr[e]);
+      const float4* cr = reinterpret_cast<const float4*>(cb + static_cast<int64_t>(c) * d_s);
+      float4 cv[8];
+#pragma unroll
+      for (int s4 = 0; s4 < 8; ++s4) cv[s4] = (s4 * 4 < d_s) ? cr[s4] : make_float4(0.f, 0.f, 0.f, 0.f);
+      float acc = 0.0f;
+#pragma unroll
+      for (int s4 = 0; s4 < 8; ++s4)
+        if (s4 * 4 < d_s) {
+          acc = fma_rn(xr[s4].x, cv[s4].x, acc);
+          acc = fma_rn(xr[s4].y, cv[s4].y, acc);
+          acc = fma_rn(xr[s4].z, cv[s4].z, acc);
+          acc = fma_rn(xr[s4].w, cv[s4].w, acc);
+        }
+      if (temperature != 1.0f) acc = acc / temperature;
+      kr[e] = composite_key(acc, static_cast<uint32_t>(c));
+    }
+  }
+  __syncthreads();
+  if (mine) {
+    int32_t* out = t.codes + (bh * t.rows + r0 + r) * top;
+    for (int e = sub; e < m; e += L) {
+      const uint64_t key = kr[e];
+      int at = 0;
+      for (int j = 0; j < m; ++j) at += kr[j] > key ? 1 : 0;
+      if (at < top) out[at] = static_cast<int32_t>(key_index(key));
+    }
+  }
+  for (int x = wave; x < R && r0 + x < t.rows; x += 4)
+    if (s_bad[x] != 0 || s_cnt[x] > kTileCap || s_cnt[x] < top)
+      exact_row_topk<TM, 1>(xb + (r0 + x) * d_s, cb, n_c, d_s, temperature, top,
+                            t.codes + (bh * t.rows + r0 + x) * top);
+}
 
 template <int TM>
 __device__ __forceinline__ void keep_top(uint64_t (&best)[TM], uint64_t key) {
@@ -1960,6 +2195,14 @@ TopkWorkspace carve_topk(void* ws, int h, int n_c) {
 }
 
 constexpr int64_t kFewTopkRows = 64;
+// Query and key rows together up to which the codebook is split over a block's waves
+// (code_topk_tile_kernel): 256-row blocks fill the CUs only past that.  Measured on
+// route_codes (16 and 4 codes): 2048 rows of 8 heads, N_c 4096 134 -> 89 us; 4096 rows
+// 135 -> 128 us (N_c 1024 114 -> 85 us); 8192 rows 175 us against 223 split.
+constexpr int64_t kTileRows = 65536;
+// ... and up to which a block takes 16 rows and not 32, which reads the codebook twice
+// as often: 2048 rows of 2 heads 44 against 48 us, 1024 rows of 8 heads 71 against 61.
+constexpr int64_t kTileNarrowRows = 8192;
 
 bool mfma_path_ok(int top, int d_s, int n_c) { return top <= 32 && d_s <= 32 && d_s % 4 == 0 && n_c <= 65535; }
 
@@ -2035,6 +2278,29 @@ int launch_mfma_pair(const float* xa, const float* xb, int64_t batch, int h, int
   return check_launch("code_topk_mfma_pair_kernel");
 }
 
+template <int NT, int TM>
+int launch_topk_tile_i(const FewTopk& ta, const FewTopk& tb, int h, const float* chat, int n_c, int d_s,
+                       float temperature, const TopkWorkspace& w, hipStream_t st) {
+  const int64_t tiles = ceil_div(ta.rows, 16 * NT);
+  const int64_t nblocks = ta.total / ta.rows * tiles * (tb.total > 0 ? 2 : 1);
+  const int64_t grid = kXcds * xcd_per(nblocks);
+  code_topk_tile_kernel<NT, TM><<<dim3(static_cast<unsigned>(grid)), 256, 0, st>>>(
+      ta, tb, h, chat, w.cbf, w.cmax_bits, n_c, d_s, temperature, tiles, nblocks);
+  return check_launch("code_topk_tile_kernel");
+}
+
+// Both tasks (tb.total = 0: only ta) have ta.rows rows per (batch, head) and top <= 32.
+int launch_topk_tile(const FewTopk& ta, const FewTopk& tb, int h, const float* chat, int n_c, int d_s,
+                     float temperature, const TopkWorkspace& w, hipStream_t st) {
+  const int top = std::max(ta.top, tb.top);
+  const bool narrow = ta.total + tb.total <= kTileNarrowRows;
+  if (top <= 16)
+    return narrow ? launch_topk_tile_i<1, 16>(ta, tb, h, chat, n_c, d_s, temperature, w, st)
+                  : launch_topk_tile_i<2, 16>(ta, tb, h, chat, n_c, d_s, temperature, w, st);
+  return narrow ? launch_topk_tile_i<1, 32>(ta, tb, h, chat, n_c, d_s, temperature, w, st)
+                : launch_topk_tile_i<2, 32>(ta, tb, h, chat, n_c, d_s, temperature, w, st);
+}
+
 // Top codes per row.  With a workspace (and top <= 32, d_s <= 32) the matrix-core
 // filter runs and the exact kernel recomputes only flagged groups; otherwise the
 // exact kernel handles every row.  `prepped` = the bf16 codebook is already in w.
@@ -2048,6 +2314,10 @@ int launch_code_topk_w(const float* xhat, int64_t batch, int h, int64_t rows, co
     const FewTopk t0{xhat, rows, batch * h * rows, top, codes};
     FewTopk none{};
     return launch_topk_few(t0, none, h, chat, n_c, d_s, temperature, st);
+  }
+  if (batch * h * rows <= kTileRows) {
+    const FewTopk t0{xhat, rows, batch * h * rows, top, codes};
+    return launch_topk_tile(t0, FewTopk{}, h, chat, n_c, d_s, temperature, w, st);
   }
   int s;
   if (top <= 4) s = launch_mfma_q<1>(xhat, batch, h, rows, chat, n_c, d_s, temperature, top, codes, w, st);
@@ -2257,10 +2527,17 @@ extern "C" int ssa_route_codes(const void* q, const void* k, int dtype, int64_t 
       return st;
   }
   if ((st = launch_normalize(codebook, static_cast<int64_t>(h_kv) * n_c, d_s, chat, s))) return st;
+  const int64_t rows = batch * h_kv * n;
+  if (rows > kFewTopkRows && 2 * rows <= kTileRows && mfma_path_ok(a, d_s, n_c) && mfma_path_ok(b, d_s, n_c)) {
+    const TopkWorkspace w = carve_topk(tws, h_kv, n_c);
+    if ((st = launch_codebook_prep(chat, h_kv, n_c, d_s, w, s))) return st;
+    const FewTopk tq{qhat, n, rows, a, q_codes}, tk{khat, n, rows, b, k_codes};
+    return launch_topk_tile(tq, tk, h_kv, chat, n_c, d_s, temperature, w, s);
+  }
   // top 16 for the queries and top 4 for the keys (config 3's a and b): both
   // screens in one launch, the keys' flag bytes after the workspace's others
   if (mf_q(a) == 4 && mf_q(b) == 1 && mfma_path_ok(a, d_s, n_c) && mfma_path_ok(b, d_s, n_c) &&
-      batch * h_kv * n > kFewTopkRows) {
+      rows > kFewTopkRows) {
     const TopkWorkspace w = carve_topk(tws, h_kv, n_c);
     uint8_t* flags_b = static_cast<uint8_t*>(tws) + topk_workspace_bytes(batch, h_kv, n, n_c);
     if ((st = launch_codebook_prep(chat, h_kv, n_c, d_s, w, s))) return st;
