@@ -238,6 +238,137 @@ __global__ __launch_bounds__(256) void index_scatter_kernel(
   }
 }
 
+// Small heads in one launch: one block per (batch, head) sorts the entries code << 16 | e
+// by code, stably, with 5-bit digits: wave w holds entries [64 w chunks, 64 (w + 1)
+// chunks) of the order so far, a lane's place in its wave is the wave's count of the
+// digit before its chunk plus the peers of its chunk below it (ballots), and a scan of
+// the 32 x 16 counts in (digit, wave) order gives the bases.  Codes out of range sort as
+// n_c, past the end.  Then postings (or the query order) are the sorted entries' keys,
+// and offsets[c] is a binary search for c.  MIN: the code of row e is its least of b.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallWaves = kSmallThreads / 64;
+constexpr int kSmallChunks = 8;
+// The four kernels above take 20 - 30 us for such a head whatever its size, nearly all of
+// it launches and latency.
+constexpr int64_t kSmallEntries = kSmallChunks * kSmallThreads;
+
+template <bool MIN>
+__global__ __launch_bounds__(kSmallThreads) void index_small_kernel(const int32_t* __restrict__ codes, int64_t n, int b,
+                                                                    int n_c, int digits,
+                                                                    int32_t* __restrict__ offsets,
+                                                                    int32_t* __restrict__ postings) {
+  extern __shared__ uint32_t sm_entries[];  // two orders of the entries
+  __shared__ int32_t cnt[kSmallWaves][32];
+  __shared__ int32_t wsum[8];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int64_t bh = blockIdx.x;
+  const int total = static_cast<int>(MIN ? n : n * b);
+  const int chunks = (total + kSmallThreads - 1) / kSmallThreads;
+  const int first = wave * 64 * chunks + lane;
+  uint32_t *src = sm_entries, *dst = sm_entries + total;
+  const int32_t* cb = codes + bh * n * b;
+  const bool quads = MIN && b % 4 == 0 && (reinterpret_cast<uintptr_t>(codes) & 15) == 0;
+  for (int e = tid; e < total; e += kSmallThreads) {
+    int32_t c;
+    if constexpr (MIN) {
+      const int32_t* ce = cb + static_cast<int64_t>(e) * b;
+      c = ce[0];
+      if (quads) {
+        for (int t = 0; t < b; t += 4) {
+          const int4 x = *reinterpret_cast<const int4*>(ce + t);
+          c = min(min(min(c, x.x), x.y), min(x.z, x.w));
+        }
+      } else {
+        for (int t = 1; t < b; ++t) c = min(c, ce[t]);
+      }
+    } else {
+      c = cb[e];
+    }
+    src[e] = (static_cast<uint32_t>(c) < static_cast<uint32_t>(n_c) ? c : n_c) << 16 | e;
+  }
+  __syncthreads();
+  const uint64_t below = (1ull << lane) - 1ull;
+  for (int dg = 0; dg < digits; ++dg) {
+    const int shift = 16 + 5 * dg;
+    if (lane < 32) cnt[wave][lane] = 0;
+    __builtin_amdgcn_wave_barrier();
+    uint32_t v[kSmallChunks];
+    int place[kSmallChunks];
+#pragma unroll
+    for (int x = 0; x < kSmallChunks; ++x) {
+      if (x >= chunks) continue;  // uniform
+      const int e = first + 64 * x;
+      const bool ok = e < total;
+      v[x] = ok ? src[e] : 0u;
+      const uint32_t d = (v[x] >> shift) & 31u;
+      uint64_t peers = __ballot(ok);
+#pragma unroll
+      for (int t = 0; t < 5; ++t) {
+        const bool set = (d >> t) & 1u;
+        const uint64_t m = __ballot(set);
+        peers &= set ? m : ~m;
+      }
+      place[x] = cnt[wave][d] + __popcll(peers & below);
+      __builtin_amdgcn_wave_barrier();
+      if (ok && (peers & below) == 0ull) cnt[wave][d] += __popcll(peers);
+      __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    int32_t own = 0, incl = 0;
+    if (tid < 32 * kSmallWaves) {
+      own = cnt[tid % kSmallWaves][tid / kSmallWaves];
+      incl = own;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int32_t y = __shfl_up(incl, o);
+        if (lane >= o) incl += y;
+      }
+      if (lane == 63) wsum[wave] = incl;
+    }
+    __syncthreads();
+    if (tid < 32 * kSmallWaves) {
+      int32_t base = incl - own;
+      for (int w = 0; w < wave; ++w) base += wsum[w];
+      cnt[tid % kSmallWaves][tid / kSmallWaves] = base;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int x = 0; x < kSmallChunks; ++x)
+      if (first + 64 * x < total && x < chunks) dst[cnt[wave][(v[x] >> shift) & 31u] + place[x]] = v[x];
+    __syncthreads();
+    uint32_t* t = src;
+    src = dst;
+    dst = t;
+  }
+  for (int e = tid; e < total; e += kSmallThreads) {
+    const uint32_t v = src[e];
+    if ((v >> 16) < static_cast<uint32_t>(n_c))
+      postings[bh * total + e] = static_cast<int32_t>(MIN ? v & 0xFFFFu : key_of(v & 0xFFFFu, b));
+  }
+  if (offsets == nullptr) return;
+  for (int c = tid; c <= n_c; c += kSmallThreads) {
+    int lo = 0, hi = total;  // the entries of codes below c
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if ((src[mid] >> 16) < static_cast<uint32_t>(c)) lo = mid + 1;
+      else hi = mid;
+    }
+    offsets[bh * (n_c + 1) + c] = lo;
+  }
+}
+
+template <bool MIN>
+int launch_index_small(const int32_t* codes, int64_t bh, int64_t n, int b, int n_c, int32_t* offsets,
+                       int32_t* postings, hipStream_t st) {
+  const size_t smem = 2 * sizeof(uint32_t) * static_cast<size_t>(MIN ? n : n * b);
+  auto kern = index_small_kernel<MIN>;
+  if (int s = reserve_lds(reinterpret_cast<const void*>(kern), smem, "index_small")) return s;
+  int digits = 1;
+  while ((n_c >> (5 * digits)) != 0) ++digits;  // (n_c itself marks a code out of range)
+  kern<<<dim3(static_cast<unsigned>(bh)), kSmallThreads, smem, st>>>(codes, n, b, n_c, digits, offsets, postings);
+  return check_launch("index_small_kernel");
+}
+
 __global__ void fill_i32_kernel(int32_t* __restrict__ p, int64_t count, int32_t v) {
   const int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
   if (e < count) p[e] = v;
@@ -258,6 +389,8 @@ int run_index(const int32_t* codes, int64_t bh, int64_t n, int b, int cstride, i
   if (n * b >= (int64_t(1) << 31))
     return fail(SSA_ERR_UNSUPPORTED, "index: n * b = %lld entries per head exceed int32 positions",
                 static_cast<long long>(n * b));
+  if (n * b <= kSmallEntries && n_c <= 16384 && cstride == b)
+    return launch_index_small<false>(codes, bh, n, b, n_c, offsets, postings, st);
   const int64_t tk = tile_keys_for(n);
   const int64_t tiles = ceil_div(n, tk);
   int code_bits = 0;
@@ -384,6 +517,7 @@ extern "C" int ssa_query_order(const int32_t* q_codes, int64_t batch, int64_t n,
   int32_t* mins = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) +
                                              query_order_hist_offsets_bytes(bh, n, n_c));
   hipStream_t st = as_stream(stream);
+  if (n <= kSmallEntries) return launch_index_small<true>(q_codes, bh, n, a, n_c, nullptr, order, st);
   const int64_t rows = bh * n;
   row_min_code_kernel<<<dim3(static_cast<unsigned>(ceil_div(rows, 256))), 256, 0, st>>>(q_codes, rows, a, mins);
   if (int s = check_launch("row_min_code_kernel")) return s;
