@@ -60,3 +60,21 @@ def test_code_tiles_last_size_and_the_next(dev, rows):
     for got, x, top in zip(kernels.route_codes(q, k, w, w, cb, 16, 4), (q, k), (16, 4)):
         ref = kernels.code_topk(kernels.route_vectors(x, w, 1), chat, top, exhaustive=True)
         assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("shift,d_s", [(0, 20), (1, 32), (3, 12)])
+def test_codebook_normalized_with_its_copy(dev, orc, shift, d_s):
+    """A codebook off 16 bytes, with a zero code, gives the codes of the normalized rows."""
+    from ssa_amd import kernels
+
+    n, h, d, n_c = 150, 2, 64, 270
+    q, k, w = randn((1, n, h, d), 41), randn((1, n, h, d), 42), randn((d_s, d), 43)
+    cb = randn((h, n_c, d_s), 44)
+    cb[0, 5] = 0.0
+    flat = torch.empty(cb.numel() + shift, device=dev)
+    cbd = flat[shift:].view(cb.shape)
+    cbd.copy_(cb)
+    chat = orc.normalize(cb.numpy())
+    for got, x, top in zip(kernels.route_codes(q.to(dev), k.to(dev), w.to(dev), w.to(dev), cbd, 16, 4), (q, k), (16, 4)):
+        ref = orc.code_topk(orc.route_vectors(x[0].numpy(), w.numpy(), 1), chat, top)
+        np.testing.assert_array_equal(got[0].cpu().numpy(), ref)
