@@ -1460,7 +1460,9 @@ __global__ __launch_bounds__(64 * kSplitWaves) void sparse_attention_split_kerne
 //              lanes (lane (q4, c16) holds keys 4 q4 + e of query c16, and step e
 //              of P.V takes keys {4 q4 + e});
 //   non-finite a V row with an infinity or NaN must not reach the rows that did
-//              not select it through 0 * inf: such a tile goes key by key.
+//              not select it through 0 * inf: such a tile goes key by key.  A NaN
+//              score stays out of the running maximum (fmaxf) but not out of the
+//              sums: while there is no other score the reference is 0.
 // Bound by the fp32 matrix cores' chains at one or two waves per SIMD: n = 2048 =
 // top_k, 8/2 heads, d = 64 takes 142 us (61 TFLOP/s) against 537 us row by row.
 constexpr int kDnWaves = 4;
@@ -1617,13 +1619,14 @@ __global__ __launch_bounds__(64 * kDnWaves, 2) void dense_f32_kernel(AttParams p
         }
         mx = rows4_reduce(mx, [](float a, float b) { return fmaxf(a, b); });
         const float mnew = fmaxf(m_run[qt], mx);
-        const bool dead = mnew == -INFINITY;
+        const bool dead = mnew == -INFINITY;  // no score yet, or none but NaN
+        const float mref = dead ? 0.0f : mnew;
         const float alpha = dead ? 1.0f : exp2f(m_run[qt] - mnew);
         m_run[qt] = mnew;
         float pr[4], ps = 0.0f;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          pr[e] = (dead || !cn[e]) ? 0.0f : exp2f(sc[qt][e] - mnew) * static_cast<float>(cn[e]);
+          pr[e] = cn[e] ? exp2f(sc[qt][e] - mref) * static_cast<float>(cn[e]) : 0.0f;
           ps += pr[e];
         }
         l_run[qt] = l_run[qt] * alpha + ps;
@@ -1689,13 +1692,14 @@ __global__ __launch_bounds__(64 * kDnWaves, 2) void dense_f32_kernel(AttParams p
     float M = -INFINITY;
 #pragma unroll
     for (int w = 0; w < kDnWaves; ++w) M = fmaxf(M, part[(w * DS::QV + qv) * DS::PROW + D]);
+    const float mref = M == -INFINITY ? 0.0f : M;
     float L = 0.0f;
     float4 O = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (int w = 0; w < kDnWaves; ++w) {
+      // (a state without a score has the weight 0 and is 0, or NaN if a key scored NaN)
       const float* pp = part + (w * DS::QV + qv) * DS::PROW;
-      if (pp[D] == -INFINITY) continue;  // no selected key in this wave's tiles
-      const float a = exp2f(pp[D] - M);
+      const float a = exp2f(pp[D] - mref);
       L += a * pp[D + 1];
       const float4 o4 = *reinterpret_cast<const float4*>(pp + 4 * x);
       O.x += a * o4.x; O.y += a * o4.y; O.z += a * o4.z; O.w += a * o4.w;

@@ -144,3 +144,50 @@ def test_dense_f32_backward_keeps_non_finite_values_apart(dev, orc, what):
         if bool((~touched).any()):
             np.testing.assert_allclose(x[~touched].numpy(), r[(~touched).numpy()], rtol=0, atol=2e-5 * np.abs(r).max())
     assert not got[0][rows].isfinite().all() and not got[1][keys].isfinite().all()
+
+
+def _torch64(q, kk, v, idx, causal, dout=None):
+    """The reference's gather -> softmax -> V (ssa/attention.py:64-113) in float64 on the
+    CPU, NaN scores included; with dout the gradients of q, k and v."""
+    q, kk, v = (t[0].double().requires_grad_(dout is not None) for t in (q, kk, v))
+    n, h_q, d = q.shape
+    h_kv = kk.shape[1]
+    head = torch.arange(h_kv)[None, :, None]
+    s = torch.einsum("nhgd,nhkd->nhgk", q.view(n, h_kv, -1, d), kk[idx[0], head]) / d**0.5
+    if causal:
+        s = s.masked_fill((idx[0] > torch.arange(n)[:, None, None])[:, :, None], -float("inf"))
+    out = torch.einsum("nhgk,nhkd->nhgd", s.softmax(-1), v[idx[0], head]).reshape(n, h_q, d)
+    return out if dout is None else torch.autograd.grad(out, (q, kk, v), dout[0].double())
+
+
+def _one_key_per_tile(n, h_kv):
+    """Row r selects the keys r mod 16 + 16 t, four times each."""
+    keys = torch.arange(n)[:, None] % 16 + 16 * torch.arange(n // 16)[None]
+    return keys.repeat(1, 4)[None, :, None].expand(1, n, h_kv, -1).contiguous()
+
+
+@pytest.mark.parametrize("g", [1, 4])
+@pytest.mark.parametrize("what", ["causal", "strided", "query"])
+def test_dense_f32_keeps_nan_scores(dev, what, g):
+    """A NaN score reaches its row's output also where its wave of the block meets no
+    other score of the row: K[16] alone in a causal row's second tile, one key a tile,
+    every key (a NaN query)."""
+    from ssa_amd import kernels
+
+    n, h_kv, d = 64, 2, 64
+    q, kk, v, idx = _case(n, h_kv, g, d, n, 71)
+    causal = what == "causal"
+    if what == "causal":
+        idx = torch.arange(n).expand(1, n, h_kv, n).contiguous()
+        kk[0, 16, 0, 5] = float("nan")
+        kk[0, 0, 1, 5] = float("nan")       # row 0 selects nothing else
+    elif what == "strided":
+        idx = _one_key_per_tile(n, h_kv)
+        kk[0, 19, 1, 0] = float("nan")
+    else:
+        q[0, 33, g, 63] = float("nan")
+    got = kernels.sparse_attention(q.to(dev), kk.to(dev), v.to(dev), idx.to(dev), None, causal)[0].cpu()
+    ref = _torch64(q, kk, v, idx, causal)
+    assert ref.isnan().any() and ref.isfinite().any()
+    # as test_dense_f32_vs_oracle
+    np.testing.assert_allclose(got.numpy(), ref.numpy(), rtol=1e-5, atol=1e-5, equal_nan=True)
