@@ -1705,11 +1705,11 @@ __global__ __launch_bounds__(64 * kDbWaves, 2) void dense_bwd_f32_kernel(BwdPara
           }
           mx = rows4_reduce(mx, [](float a, float b) { return fmaxf(a, b); });
           const float mnew = fmaxf(m_run[qt], mx);
-          const bool dead = mnew == -INFINITY;
+          const bool dead = mnew == -INFINITY;  // no score yet, or none but NaN
+          const float mref = dead ? 0.0f : mnew;
           float ps = 0.0f;
 #pragma unroll
-          for (int e = 0; e < 4; ++e)
-            ps += (dead || !cn[e]) ? 0.0f : exp2f(sc[e] - mnew) * static_cast<float>(cn[e]);
+          for (int e = 0; e < 4; ++e) ps += cn[e] ? exp2f(sc[e] - mref) * static_cast<float>(cn[e]) : 0.0f;
           l_run[qt] = l_run[qt] * (dead ? 1.0f : exp2f(m_run[qt] - mnew)) + ps;
           m_run[qt] = mnew;
         }
@@ -1728,10 +1728,11 @@ __global__ __launch_bounds__(64 * kDbWaves, 2) void dense_bwd_f32_kernel(BwdPara
       float M = -INFINITY, L = 0.0f;
 #pragma unroll
       for (int w = 0; w < kDbWaves; ++w) M = fmaxf(M, s_st[w][tid][0]);
+      const float mref = M == -INFINITY ? 0.0f : M;
+      // (a state without a score has the weight 0 and is 0, or NaN if a key scored NaN)
 #pragma unroll
-      for (int w = 0; w < kDbWaves; ++w)
-        if (s_st[w][tid][0] != -INFINITY) L += exp2f(s_st[w][tid][0] - M) * s_st[w][tid][1];
-      s_m[tid] = M == -INFINITY ? 0.0f : M;
+      for (int w = 0; w < kDbWaves; ++w) L += exp2f(s_st[w][tid][0] - mref) * s_st[w][tid][1];
+      s_m[tid] = mref;
       s_inv[tid] = L > 0.0f ? 1.0f / L : (L == 0.0f ? 0.0f : L);  // (a NaN stays one)
     }
     __syncthreads();

@@ -191,3 +191,31 @@ def test_dense_f32_keeps_nan_scores(dev, what, g):
     assert ref.isnan().any() and ref.isfinite().any()
     # as test_dense_f32_vs_oracle
     np.testing.assert_allclose(got.numpy(), ref.numpy(), rtol=1e-5, atol=1e-5, equal_nan=True)
+
+
+def _check_backward(dev, q, kk, v, idx, causal):
+    from ssa_amd import kernels
+
+    dout = randn(q.shape, 85)
+    args = [t.to(dev) for t in (q, kk, v, idx)]
+    out = kernels.sparse_attention(*args, None, causal)
+    got = kernels.sparse_attention_backward(*args, out, dout.to(dev), None, causal)
+    for x, ref in zip(got, _torch64(q, kk, v, idx, causal, dout)):
+        # as test_dense_f32_backward_vs_oracle
+        atol = 2e-5 * float(ref[ref.isfinite()].abs().max())
+        np.testing.assert_allclose(x[0].cpu().numpy(), ref.numpy(), rtol=0, atol=atol, equal_nan=True)
+
+
+@pytest.mark.parametrize("g", [1, 4])
+@pytest.mark.parametrize("what", ["strided", "query"])
+def test_dense_f32_backward_keeps_nan_scores(dev, what, g):
+    """A NaN score makes its row's whole softmax NaN, and with it dv and dk of every key
+    that the row selects, also where its wave meets no other score of the row."""
+    n, h_kv, d = 64, 2, 64
+    q, kk, v, idx = _case(n, h_kv, g, d, 24, 81)
+    if what == "strided":
+        idx = _one_key_per_tile(n, h_kv)
+        kk[0, 19, 1, 0] = float("nan")
+    else:
+        q[0, 33, g, 63] = float("nan")
+    _check_backward(dev, q, kk, v, idx, False)
