@@ -1668,9 +1668,12 @@ __global__ __launch_bounds__(64 * kDbWaves, 2) void dense_bwd_f32_kernel(BwdPara
     }
     return s;
   };
+  // (query vectors past the block's R g select nothing: their zeros against a K with an
+  // infinity would give the row R - 1's keys a NaN)
   auto counts = [&](int qt, int tile, uint32_t (&cn)[4]) {
-    const uint2 c2 =
+    uint2 c2 =
         *reinterpret_cast<const uint2*>(reinterpret_cast<const uint16_t*>(kw.cnt) + crow[qt] + tile * kKeyTile);
+    if (16 * qt + c16 >= R * g) c2 = make_uint2(0u, 0u);
     cn[0] = c2.x & 0xFFFFu; cn[1] = c2.x >> 16; cn[2] = c2.y & 0xFFFFu; cn[3] = c2.y >> 16;
   };
 

@@ -219,3 +219,13 @@ def test_dense_f32_backward_keeps_nan_scores(dev, what, g):
     else:
         q[0, 33, g, 63] = float("nan")
     _check_backward(dev, q, kk, v, idx, False)
+
+
+def test_dense_f32_backward_unused_query_vectors_add_nothing(dev):
+    """g = 3 leaves query vectors of a block without a row: they must not meet a key whose
+    infinity (a score of -inf for the rows that select it) would make them NaN."""
+    n, h_kv, g, d, at = 80, 2, 3, 64, 11
+    q, kk, v, idx = _case(n, h_kv, g, d, 24, 91)
+    q[0, :, :, 7] = q[0, :, :, 7].abs() + 0.1
+    kk[0, at, 1, 7] = -float("inf")
+    _check_backward(dev, q, kk, v, idx, False)
