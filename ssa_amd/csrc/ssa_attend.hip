@@ -16,6 +16,8 @@
 #include "ssa_internal.h"
 #include "ssa_rows.h"
 
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace ssa {
@@ -1715,17 +1717,49 @@ __global__ __launch_bounds__(64 * kDnWaves, 2) void dense_f32_kernel(AttParams p
   }
 }
 
-// Taken while n * max(g, 2) <= 16 top_k: its time grows with n g, the row
-// kernel's with top_k (a row's products cost the same for 1 to 4 heads there).
-// Random selections on MI355X, us, row kernel / this one:
-//   d = 64   8 kv heads, g = 1:  n = 2048, k = 512: 453 / 222;  k = 256: 238 / 165;  k = 128: 131 / 144
-//            2 kv heads, g = 4:  n = 2048, k = 2048: 657 / 143;  k = 512: 152 / 115;  k = 256: 79 / 112
-//            2 kv heads, g = 8:  n = 2048, k = 2048: 652 / 242;  k = 512: 164 / 219
-//   d = 128  2 kv heads, g = 4:  n = 2048, k = 2048: 1369 / 255;  k = 512: 341 / 237;  k = 256: 184 / 231
+// Taken where the estimate below finds it faster than the row kernel, and only while
+// n * max(g, 2) <= 16 top_k (past that the row kernel wins or was not measured).  Both
+// times (us) are a call's floor and, joined as the cube root of their cubes, what one
+// row or block takes alone and what all of them take on a full GPU:
+//   row kernel   its slots one chunk after the other; all rows' slots (more for groups
+//                of over 4 and over 8 heads);
+//   this one     a wave's tiles, and the index lists its block's rows read again for
+//                each window of keys; all blocks' tiles, and per row the marks and the
+//                lists (top_k entries a window: this part grows with n^2 / LDS).
+// The constants are fitted to 1100 random selections on MI355X (1 to 16 heads a group, n
+// = 203 to 16384, 1 to 90000 rows; within 12% rms).  Row kernel / this one, us:
+//   d = 64   8 kv heads, g = 1:  n = 2048, k = 256: 236 / 162;  k = 1024: 870 / 325
+//                                n = 4096, k = 512: 859 / 799;  n = 8192, k = 1024: 3341 / 4432
+//                                n = 16384, k = 2048: 13.2 / 29.5 ms (29 windows)
+//            2 kv heads, g = 4:  n = 2048, k = 2048: 654 / 143;  k = 512: 149 / 114
+//                                n = 8192, k = 2048: 1687 / 1929;  k = 8192: 7002 / 3217
+//            1 kv head, g = 8:   n = 4096, k = 2048: 627 / 433;  n = 16384, k = 8192: 9327 / 7590
+//            8 kv heads, g = 1, n = 8192, k = 1024: 1 row 105 / 176;  128 rows 119 / 354
+//   d = 128  8 kv heads, g = 1:  n = 16384, k = 2048: 44.6 / 24.1 ms
+//            2 kv heads, g = 4:  n = 2048, k = 512: 338 / 235;  n = 16384, k = 4096: 21.8 / 14.6 ms
+//            8 kv heads, g = 1, n = 2048, k = 256: 1 row 44 / 71;  128 rows 50 / 94;  512 rows 182 / 95
 // Two 16-query tiles a block at d = 64 once that leaves 512 blocks (2 waves a
 // SIMD); at d = 128 two do not fit the registers.
 constexpr int kDnKeysPerSlot = 16;
 constexpr int64_t kDnTwoTiles = 32 * 512;  // query vectors
+
+bool dense_f32_faster(const AttParams& p) {
+  if (p.top_k >= (1 << 16) || p.n * max(p.g, 2) > static_cast<int64_t>(p.top_k) * kDnKeysPerSlot) return false;
+  const bool wide = p.d == 128;
+  const int qt = !wide && p.rows * p.g >= kDnTwoTiles ? 2 : 1;
+  const int R = 16 * qt / p.g;
+  const double n = static_cast<double>(p.n), k = p.top_k, rows = static_cast<double>(p.rows);
+  const double windows = static_cast<double>(ceil_div(p.n, key_window(p.n, R, kDnCountBytes)));
+  const double vectors = 16.0 * qt * static_cast<double>((p.rows / p.n_q) * ceil_div(p.n_q, R));
+  const auto both = [](double alone, double full) { return std::cbrt(alone * alone * alone + full * full * full); };
+  const double slot_ps = wide ? (p.g <= 4 ? 167 : p.g <= 8 ? 193 : 213) : (p.g <= 4 ? 57 : 85);
+  const double row = (wide ? 5.7 : 4.8) + both((wide ? 0.158 : 0.101) * k, 1e-6 * slot_ps * rows * k);
+  const double lists = 0.25 * static_cast<double>(std::min<int64_t>(R, p.n_q)) * windows * k;  // entries a wave reads
+  const double tiles = (wide ? 6.8 : 3.35) * vectors * n, marks = (2.4 * (windows - 1.0) + 6.3) * rows * k;
+  const double dense = (wide ? 7.2 : 5.6) + both((wide ? 0.0328 : 0.019) * n + 0.0048 * lists, 1e-6 * (tiles + marks));
+  // (past four windows the lists no longer stay in L2 and the estimate is low)
+  return dense < row * (windows > 4.0 ? 0.92 : wide ? 0.97 : 1.06);
+}
 
 template <int D, int QT>
 int launch_dense_f32(const AttParams& p, hipStream_t st) {
@@ -1783,7 +1817,7 @@ int launch_att_d(const AttParams& p, hipStream_t st) {
     }
   }
   if constexpr (sizeof(T) == 4 && (D == 64 || D == 128)) {
-    if (p.blk_log2 == 0 && p.d == D && p.top_k < (1 << 16) && p.n * max(p.g, 2) <= static_cast<int64_t>(p.top_k) * kDnKeysPerSlot) {
+    if (p.blk_log2 == 0 && p.d == D && dense_f32_faster(p)) {
       const int64_t qvs = p.rows * p.g;
       if (D == 64 && qvs >= kDnTwoTiles) return launch_dense_f32<D, (D == 64 ? 2 : 1)>(p, st);
       return launch_dense_f32<D, 1>(p, st);

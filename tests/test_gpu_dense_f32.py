@@ -161,9 +161,9 @@ def _torch64(q, kk, v, idx, causal, dout=None):
 
 
 def _one_key_per_tile(n, h_kv):
-    """Row r selects the keys r mod 16 + 16 t, four times each."""
+    """Row r selects the keys r mod 16 + 16 t, eight times each."""
     keys = torch.arange(n)[:, None] % 16 + 16 * torch.arange(n // 16)[None]
-    return keys.repeat(1, 4)[None, :, None].expand(1, n, h_kv, -1).contiguous()
+    return keys.repeat(1, 8)[None, :, None].expand(1, n, h_kv, -1).contiguous()
 
 
 @pytest.mark.parametrize("g", [1, 4])
@@ -191,6 +191,28 @@ def test_dense_f32_keeps_nan_scores(dev, what, g):
     assert ref.isnan().any() and ref.isfinite().any()
     # as test_dense_f32_vs_oracle
     np.testing.assert_allclose(got.numpy(), ref.numpy(), rtol=1e-5, atol=1e-5, equal_nan=True)
+
+
+@pytest.mark.parametrize("d,g,n,k,n_q,i64", [
+    (64, 1, 2500, 320, 1, False),     # few rows: each gathers its own keys
+    (64, 1, 2500, 320, 700, True),
+    (128, 2, 1300, 600, 40, True),    # tiles, 40 of 1300 positions
+    (64, 1, 2500, 2500, 64, False)])  # three windows, every key
+def test_dense_f32_rows_at_the_end_vs_oracle(dev, orc, d, g, n, k, n_q, i64):
+    """A block of n_q query rows at the last positions, on both sides of the rule that
+    weighs the tiles against the rows' gathers."""
+    from ssa_amd import kernels
+
+    q, kk, v, idx = _case(n, 1, g, d, k, 101)
+    rows = np.arange(n - n_q, n)
+    idx = idx[:, n - n_q:] if i64 else idx[:, n - n_q:].to(torch.int32)
+    flag = torch.zeros(1, dtype=torch.int32, device=dev)
+    got = kernels.sparse_attention(q[:, n - n_q:].to(dev), kk.to(dev), v.to(dev), idx.to(dev), None, True,
+                                   error_flag=flag)
+    assert int(flag.item()) == 0
+    ref = orc.sparse_attention(f32(q[0]), f32(kk[0]), f32(v[0]), idx[0].to(torch.int64).numpy(), causal=True, rows=rows)
+    # as test_dense_f32_vs_oracle
+    np.testing.assert_allclose(got[0].cpu().numpy(), ref, rtol=1e-5, atol=1e-5)
 
 
 def _check_backward(dev, q, kk, v, idx, causal):
