@@ -1905,23 +1905,46 @@ __global__ __launch_bounds__(64 * kDbWaves, 2) void dense_bwd_f32_kernel(BwdPara
   }
 }
 
-// Taken while n <= 12 top_k (d = 64) or 5 top_k (d = 128): its time grows with n,
-// the row kernel's with top_k, both with g.  Random selections on MI355X, us, row
-// kernel / this one:
-//   d = 64   8 kv heads, g = 1:  n = 2048, k = 256: 2197 / 667;  k = 128: 1098 / 568;  k = 64: 564 / 603
-//            2 kv heads, g = 4:  n = 2048, k = 256: 990 / 497;   k = 128: 506 / 505
-//            2 kv heads, g = 8:  n = 1024, k = 128: 667 / 264;   n = 2048, k = 128: 937 / 936
-//   d = 128  2 kv heads, g = 4:  n = 2048, k = 512: 2568 / 1721; k = 256: 1293 / 1716
-//            8 kv heads, g = 1:  n = 1024, k = 128: 1157 / 520
+// Taken while n <= 12 top_k (d = 64) or 5 top_k (d = 128), past which nothing was
+// measured or the row kernel wins, and where a row costs less here than there.  A row
+// here: its share of the block's tiles, for every key, and its list once more for each
+// window of keys after the first (both passes; that part grows with n^2 / LDS).  A row
+// of the row kernel: its slots, each dearer with the heads and with the register
+// arrays of 4, 8 and 16 of them; with at most two rows a SIMD half as much again.
+// Random selections on MI355X, us, row kernel / this one:
+//   d = 64   8 kv heads, g = 1:  n = 2048, k = 171: 1464 / 644;  n = 8192, k = 683: 20.4 / 12.5 ms
+//            1 kv head, g = 1:   n = 16384, k = 1366: 11.3 / 9.6 ms;  n = 32768, k = 2731: 43 / 65 ms
+//                                (103 windows);  g = 2, n = 32768, k = 2731: 46 / 45 ms
+//            2 kv heads, g = 4:  n = 2048, k = 171: 661 / 488;  n = 16384, k = 1366: 33.9 / 29.2 ms
+//            1 kv head, g = 8:   n = 4096, k = 342: 2455 / 1852
+//   d = 128  8 kv heads, g = 1:  n = 1024, k = 205: 1741 / 522
+//            2 kv heads, g = 4:  n = 2048, k = 410: 2055 / 1713;  n = 16384, k = 3277: 100 / 105 ms
+//            1 kv head, g = 8:   n = 2048, k = 410: 2323 / 1696;  n = 4096, k = 820: 5947 / 6563
+//            1 kv head, n = 4096, k = 820:  g = 7: 5314 / 6514;  g = 10: 11.1 / 12.6 ms;  g = 13: 13.7 / 12.6 ms
 constexpr int kDbKeysPerSlot64 = 12, kDbKeysPerSlot128 = 5;
 constexpr int64_t kDbTwoTiles = 32 * 256;  // query vectors
+constexpr int64_t kDbFewRows = 2048;
+
+bool dense_bwd_f32_faster(const BwdParams& p) {
+  const bool wide = p.d == 128;
+  if (p.top_k >= (1 << 16) || p.n > static_cast<int64_t>(p.top_k) * (wide ? kDbKeysPerSlot128 : kDbKeysPerSlot64))
+    return false;
+  const int qt = !wide && p.rows * p.g >= kDbTwoTiles ? 2 : 1;
+  const int R = 16 * qt / p.g;
+  const double windows = static_cast<double>(ceil_div(p.n, key_window(p.n, R, kDbCountBytes)));
+  // picoseconds on a full GPU: per row and slot there; per query vector and key, per entry read here
+  static const double slot64[9] = {0, 500, 620, 620, 780, 1000, 1200, 1400, 1540};
+  static const double slot128[9] = {0, 850, 980, 1000, 1020, 1330, 1600, 1620, 1800};
+  const double slot = p.g <= 8 ? (wide ? slot128 : slot64)[p.g] : (wide ? 770.0 + 255.0 * p.g : 240.0 * p.g);
+  const double tiles = (wide ? 50.0 : 13.0) * 16 * qt / R * static_cast<double>(p.n);
+  return tiles + 6.3 * (windows - 1.0) * p.top_k <= slot * p.top_k * (p.rows <= kDbFewRows ? 1.5 : 1.0);
+}
 
 bool dense_bwd_f32_ok(const BwdParams& p) {
   const auto rows16 = [](const void* x, int64_t sb, int64_t sn, int64_t sh) {
     return reinterpret_cast<uintptr_t>(x) % 16 == 0 && sb % 4 == 0 && sn % 4 == 0 && sh % 4 == 0;
   };
-  return (p.d == 64 || p.d == 128) && p.top_k < (1 << 16) &&
-         p.n <= static_cast<int64_t>(p.top_k) * (p.d == 64 ? kDbKeysPerSlot64 : kDbKeysPerSlot128) && rows16(p.k, p.k_sb, p.k_sn, p.k_sh) &&
+  return (p.d == 64 || p.d == 128) && dense_bwd_f32_faster(p) && rows16(p.k, p.k_sb, p.k_sn, p.k_sh) &&
          rows16(p.v, p.v_sb, p.v_sn, p.v_sh) && reinterpret_cast<uintptr_t>(p.dq) % 16 == 0;
 }
 

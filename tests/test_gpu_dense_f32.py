@@ -251,3 +251,23 @@ def test_dense_f32_backward_unused_query_vectors_add_nothing(dev):
     q[0, :, :, 7] = q[0, :, :, 7].abs() + 0.1
     kk[0, at, 1, 7] = -float("inf")
     _check_backward(dev, q, kk, v, idx, False)
+
+
+@pytest.mark.parametrize("g", [9, 13])
+def test_dense_f32_backward_on_both_sides_of_its_rule(dev, g):
+    """d = 128, n / k just under 5, more rows than the rule counts as few: nine heads go
+    row by row, thirteen by key tiles."""
+    from ssa_amd import kernels
+
+    n, d, k = 2100, 128, 430
+    q, kk, v, idx = (t.to(dev) for t in _case(n, 1, g, d, k, 111))
+    dout = randn((1, n, g, d), 115).to(dev)
+    out = kernels.sparse_attention(q, kk, v, idx)
+    got = kernels.sparse_attention_backward(q, kk, v, idx, out, dout)
+    q64, k64, v64 = (t[0].double().transpose(0, 1).contiguous().requires_grad_(True) for t in (q, kk, v))
+    off = torch.ones(n, n, dtype=torch.bool, device=dev).scatter_(1, idx[0, :, 0], False)
+    p = (torch.matmul(q64, k64[0].t().contiguous()) / d**0.5).masked_fill(off, -float("inf")).softmax(-1)
+    ref = torch.autograd.grad(torch.matmul(p, v64[0]), (q64, k64, v64), dout[0].double().transpose(0, 1))
+    for x, r in zip(got, ref):
+        # as test_dense_f32_backward_vs_oracle
+        assert float((x[0] - r.transpose(0, 1)).abs().max()) <= 2e-5 * float(r.abs().max())
