@@ -249,11 +249,28 @@ __global__ __launch_bounds__(256) void index_scatter_kernel(
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallWaves = kSmallThreads / 64;
 constexpr int kSmallChunks = 8;
-// Up to 8192 entries a head: the four kernels above take 27 us there, nearly all of it
-// latency; this one 7 us for 812 entries, 15 us for 4096, 22 us against 32 for 8192 (the
-// order of 8192 rows by 16 codes 35 against 47 us).  Bound by the ballots of one CU, so it
-// grows with the entries, which the tiles of the other kernels spread over the chip.
+// Bound by the ballots of one CU, so it grows with the entries, which the tiles of the
+// other kernels spread over the chip where there are few heads.  Those four kernels (and
+// row_min_code_kernel) / this one, us:
+//   index   8 heads, 2048 entries (b = 4), N_c 2048: 22 / 12;  8192: 30 / 22;  N_c 16384: 121 / 35
+//           8192 entries of b = 1 (more and smaller tiles there), 8 heads: N_c 512: 14.8 / 15.8;
+//           N_c 2048: 19.8 / 22.1;  N_c 4096: 24.5 / 23.7;  256 heads, N_c 512: 32 / 17
+//   order   (here with its minima, one CU reading a head's n a codes)
+//           8 heads, N_c 1024, n = 4096: 16 codes 20 / 17, 32 codes 23 / 28;  n = 8192:
+//           4 codes 19 / 21, 16 codes 21 / 29;  N_c 4096: 16 codes 29 / 28, 32 codes 31 / 49
+//           32 heads, n = 4096, 32 codes, N_c 1024: 34 / 28;  n = 8192, 64 codes: 85 / 97
+//           256 heads, n = 4096, 32 codes, N_c 1024: 521 / 61
+// so few heads of more than 4096 keys take it with large codebooks only, and the codes
+// of an order are limited per head, the more the heads the less.
 constexpr int64_t kSmallEntries = kSmallChunks * kSmallThreads;
+// (entries are packed with codes of 16 bits; the backward's index by prefix length has
+// top_k + 1 of them)
+inline bool index_small_ok(int64_t bh, int64_t n, int b, int n_c) {
+  return n * b <= kSmallEntries && n_c <= 16384 && (n <= 4096 || n_c >= 4096 || bh >= 32);
+}
+inline bool order_small_ok(int64_t bh, int64_t n, int a, int n_c) {
+  return index_small_ok(bh, n, 1, n_c) && n * a <= (n_c >= 4096 ? 131072 : 65536) * (bh < 8 ? 1 : bh / 8);
+}
 
 template <bool MIN>
 __global__ __launch_bounds__(kSmallThreads) void index_small_kernel(const int32_t* __restrict__ codes, int64_t n, int b,
@@ -392,7 +409,7 @@ int run_index(const int32_t* codes, int64_t bh, int64_t n, int b, int cstride, i
   if (n * b >= (int64_t(1) << 31))
     return fail(SSA_ERR_UNSUPPORTED, "index: n * b = %lld entries per head exceed int32 positions",
                 static_cast<long long>(n * b));
-  if (n * b <= kSmallEntries && n_c <= 16384 && cstride == b)
+  if (index_small_ok(bh, n, b, n_c))
     return launch_index_small<false>(codes, bh, n, b, n_c, offsets, postings, st);
   const int64_t tk = tile_keys_for(n);
   const int64_t tiles = ceil_div(n, tk);
@@ -520,7 +537,8 @@ extern "C" int ssa_query_order(const int32_t* q_codes, int64_t batch, int64_t n,
   int32_t* mins = reinterpret_cast<int32_t*>(static_cast<char*>(workspace) +
                                              query_order_hist_offsets_bytes(bh, n, n_c));
   hipStream_t st = as_stream(stream);
-  if (n <= kSmallEntries) return launch_index_small<true>(q_codes, bh, n, a, n_c, nullptr, order, st);
+  if (order_small_ok(bh, n, a, n_c))
+    return launch_index_small<true>(q_codes, bh, n, a, n_c, nullptr, order, st);
   const int64_t rows = bh * n;
   row_min_code_kernel<<<dim3(static_cast<unsigned>(ceil_div(rows, 256))), 256, 0, st>>>(q_codes, rows, a, mins);
   if (int s = check_launch("row_min_code_kernel")) return s;

@@ -51,3 +51,19 @@ def test_query_order_of_small_heads(dev, n, a, n_c, shift):
     q.copy_(torch.from_numpy(codes))
     got = kernels.query_order(q, n_c).cpu().numpy()
     np.testing.assert_array_equal(got, np.argsort(codes.min(-1), axis=-1, kind="stable"))
+
+
+@pytest.mark.parametrize("bh,n,a,n_c", [
+    (2, 4096, 16, 512), (2, 4097, 15, 512), (2, 4096, 17, 512), (2, 8192, 16, 4095), (2, 8192, 16, 4096),
+    (2, 8192, 17, 4096), (31, 8192, 1, 512), (32, 8192, 1, 512), (16, 4096, 33, 1000)])
+def test_query_order_on_both_sides_of_its_rule(dev, bh, n, a, n_c):
+    """One launch, or the minima and the four kernels: by the rows, codes and heads."""
+    from ssa_amd import kernels
+
+    codes = np.random.default_rng(n + a + n_c).integers(0, n_c, (1, bh, n, a)).astype(np.int32)
+    got = kernels.query_order(torch.from_numpy(codes).to(dev), n_c).cpu().numpy()
+    np.testing.assert_array_equal(got, np.argsort(codes.min(-1), axis=-1, kind="stable"))
+    off, post = (t.cpu().numpy() for t in kernels.build_index(torch.from_numpy(codes[..., :1].copy()).to(dev), n_c))
+    np.testing.assert_array_equal(post, np.argsort(codes[..., 0], axis=-1, kind="stable"))
+    for h in range(bh):
+        np.testing.assert_array_equal(off[0, h], np.searchsorted(np.sort(codes[0, h, :, 0]), np.arange(n_c + 1)))
