@@ -86,6 +86,13 @@ __device__ __forceinline__ int wave_incl_scan(int x) {
   return v;
 }
 
+// LDS hand-off between lanes of one wave (each wave owns its LDS slices).
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
 // fp32 fused multiply-add, single rounding (v_fma_f32).
 __device__ __forceinline__ float fma_rn(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 

@@ -311,7 +311,7 @@ __global__ __launch_bounds__(kSmallThreads) void index_small_kernel(const int32_
   for (int dg = 0; dg < digits; ++dg) {
     const int shift = 16 + 5 * dg;
     if (lane < 32) cnt[wave][lane] = 0;
-    __builtin_amdgcn_wave_barrier();
+    wave_lds_sync();
     uint32_t v[kSmallChunks];
     int place[kSmallChunks];
 #pragma unroll
@@ -329,9 +329,9 @@ __global__ __launch_bounds__(kSmallThreads) void index_small_kernel(const int32_
         peers &= set ? m : ~m;
       }
       place[x] = cnt[wave][d] + __popcll(peers & below);
-      __builtin_amdgcn_wave_barrier();
+      wave_lds_sync();
       if (ok && (peers & below) == 0ull) cnt[wave][d] += __popcll(peers);
-      __builtin_amdgcn_wave_barrier();
+      wave_lds_sync();
     }
     __syncthreads();
     int32_t own = 0, incl = 0;

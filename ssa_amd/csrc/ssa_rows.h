@@ -200,13 +200,6 @@ __device__ __forceinline__ void barrier_keep_loads() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
-// LDS hand-off between lanes of one wave (each wave owns its LDS slices).
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
 // ---- key windows: how often each of a few rows selects each key ----------------
 //
 // The fp32 kernels that run many query vectors against consecutive keys
