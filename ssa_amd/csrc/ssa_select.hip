@@ -872,7 +872,9 @@ __global__ __launch_bounds__(kSelThreads) void select_kernel(SelParams p, const 
 // A row with more than kFewCap candidates goes on as select_row, on the first 256
 // threads (the other waves end).  Same results.
 // Eight rows over a cache of 32700 keys (32/8 heads, 16 codes, k = 512): 15 us against
-// 45 us; the decoding step 79 -> 51 us.
+// 45 us; the decoding step 79 -> 51 us.  256 rows, select_kernel / this one, us (k = 512):
+// 2000 candidates 48 / 17, 4100 postings of 32 codes 93 / 28, 130 candidates (filler
+// mostly) 7.5 / 8.1, 8200 (past the cap) 167 / 173.
 constexpr int kFewThreads = 1024;
 constexpr int kFewCap = 2048;
 constexpr int64_t kFewRows = 256;  // one block per CU
@@ -938,7 +940,8 @@ __global__ __launch_bounds__(kFewThreads) void select_few_kernel(SelParams p, co
   if constexpr (kMatrix) stage_queries<GMAX, D, kFewThreads>(q0, p.q_sh, p.g, qs, tid);
   __syncthreads();
   const int R = s_start[p.nseg];
-  for (int base = 0; base < R; base += kFewThreads) {
+  // (a wave that sees the list overrun stops: the row starts over below.  s_cnt only grows)
+  for (int base = 0; base < R && s_cnt <= kFewCap; base += kFewThreads) {
     const int pidx = base + tid;
     bool fresh = false;
     int32_t j = 0;
