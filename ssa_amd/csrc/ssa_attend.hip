@@ -1248,8 +1248,8 @@ __global__ __launch_bounds__(64 * kPfxWaves, 2) void prefix_attention_kernel(Att
 //           in the prefix pass; only the query's own block needs the causal mask.
 // bf16, g <= 8, d = 64 / 128, bs >= 32 (a chunk lies inside one block); smaller
 // blocks keep the row kernel, which gathers each row's keys by itself.
-// QT = 2 from 128 query vectors per block on: each K/V fragment read from LDS
-// then serves two tiles.
+// QT = 2 past 64 query vectors per block: each K/V fragment read from LDS then
+// serves two tiles.
 // Bound by the softmax's VALU work beside the MFMAs (P.V runs twice, for P's hi
 // and lo parts).  n = 32768, 32/8 heads, d = 128, bs = 64, 16 blocks a query
 // block: 0.80 ms (344 TFLOP/s) against 5.55 ms with the row kernel, which
@@ -1773,6 +1773,20 @@ int launch_dense_f32(const AttParams& p, hipStream_t st) {
   return check_launch("dense_f32_kernel");
 }
 
+// Small block-granular calls go row by row: with a wave for every row and a SIMD for
+// every wave the row kernel's chain of chunks is the shorter one (it shares no barrier
+// and each wave has one query tile).  Row kernel / block_attention_kernel, us, d = 128
+// unless noted (nb blocks of bs keys):
+//   two tiles a wave   8/1 heads, n = 1024, bs = 64:  nb = 1: 6.6 / 8.5;  4: 13.2 / 15.1;  16: 40 / 40
+//                      32/8 heads, n = 256, bs = 32:  nb = 1: 6.1 / 7.3;  4: 11.7 / 10.4
+//                      8/2 heads, d = 64, n = 1024:   bs = 64, nb = 1: 5.9 / 6.4;  4: 12.6 / 11.1
+//   one                8/8 heads, n = 65, bs = 64, nb = 1: 5.8 / 6.4;  n = 256: 8.1 / 6.4
+//                      2/2 heads, d = 64, n = 256, bs = 32:  nb = 1: 4.0 / 4.4;  4: 6.6 / 5.9
+constexpr int64_t kBlkFewRows = 1024;  // one a SIMD
+inline bool block_rows_faster(const AttParams& p, int qt) {
+  return p.rows <= kBlkFewRows * qt && (p.top_k <= 64 || (qt == 2 && p.rows <= kBlkFewRows));
+}
+
 template <typename T, int D>
 int launch_att_d(const AttParams& p, hipStream_t st) {
   const int64_t blocks = ceil_div(p.rows, kAttWaves);
@@ -1805,10 +1819,12 @@ int launch_att_d(const AttParams& p, hipStream_t st) {
         const int64_t qvs = static_cast<int64_t>(p.g) << p.blk_log2;
         const int qt = qvs > 16 * kBlkWaves ? 2 : 1;
         const int64_t nblk = (p.rows / p.n_q) * p.nbk * ceil_div(qvs, 16 * qt * kBlkWaves);
-        const dim3 bgrid(static_cast<unsigned>(kXcds * xcd_per(nblk)));
-        if (qt == 2) block_attention_kernel<D, 2><<<bgrid, 64 * kBlkWaves, 0, st>>>(p);
-        else block_attention_kernel<D, 1><<<bgrid, 64 * kBlkWaves, 0, st>>>(p);
-        return check_launch("block_attention_kernel");
+        if (!block_rows_faster(p, qt)) {
+          const dim3 bgrid(static_cast<unsigned>(kXcds * xcd_per(nblk)));
+          if (qt == 2) block_attention_kernel<D, 2><<<bgrid, 64 * kBlkWaves, 0, st>>>(p);
+          else block_attention_kernel<D, 1><<<bgrid, 64 * kBlkWaves, 0, st>>>(p);
+          return check_launch("block_attention_kernel");
+        }
       }
       const dim3 grid(static_cast<unsigned>(kXcds * xcd_per(ceil_div(p.rows, kMfWaves))));
       if (p.blk_log2 > 0) sparse_attention_mfma_kernel<D, true><<<grid, 64 * kMfWaves, 0, st>>>(pr);
