@@ -54,3 +54,23 @@ def test_route_codes_queries_and_keys_in_one_launch(dev, orc):
     for x, w, g, top, got in ((q, wq, h_q // h_kv, 8, qc), (k, wk, 1, 4, kc)):
         ref = orc.code_topk(orc.route_vectors(f32(x[0]), f32(w), g), chat, top)
         np.testing.assert_array_equal(got[0].cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("d,group", [(64, 1), (128, 3)])
+def test_route_vectors_denormals_keep_their_bits(dev, orc, dtype, d, group):
+    """Rows that are denormal, whose products are, and whose sums pass through the denormals."""
+    from ssa_amd import kernels
+
+    n, h_out, d_s = 160, 2, 32
+    scale = torch.tensor([1.0, 1e-37, 1e-38, 3e-39, 2e-40, 1e-20])[torch.arange(n) % 6]
+    x = (randn((1, n, h_out * group, d), 21) * scale[None, :, None, None]).to(dtype)
+    w = randn((d_s, d), 22)
+    w[1] *= 1e-20                                   # 1e-20 against 1e-20: products are denormal
+    w[2] *= 1e-39                                   # itself denormal
+    w[3, ::2] = 1.0
+    w[3, 1::2] = -1.0                               # sums that cancel down to them
+    got = kernels.route_vectors(x.to(dev), w.to(dev), group).cpu().numpy()
+    xs = f32(x)
+    assert (np.abs(xs[(xs != 0)]) < 1.1e-38).any()
+    np.testing.assert_array_equal(got[0], orc.route_vectors(xs[0], f32(w), group))
