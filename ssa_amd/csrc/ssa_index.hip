@@ -30,20 +30,15 @@ int64_t tile_keys_for(int64_t n) {
   return tk < 1024 ? 1024 : tk;
 }
 
-// Entry e = j*b + r of a head is code r of key j, stored at j*cstride + r
-// (cstride = b for k_codes; the query order reads each row's smallest code
-// with b = 1, cstride = 1).  Entries of a head number below 2^31 (run_index checks), so the
+// Entry e = j*b + r of a head is code r of key j (the query order has one code a row:
+// its smallest).  Entries of a head number below 2^31 (run_index checks), so the
 // division is 32-bit: no branches between a load's address and its use.
 __device__ __forceinline__ uint32_t key_of(int64_t e, int b) {
   return static_cast<uint32_t>(e) / static_cast<uint32_t>(b);
 }
-__device__ __forceinline__ int64_t code_at(int64_t e, int b, int cstride) {
-  const uint32_t j = key_of(e, b);
-  return static_cast<int64_t>(j) * cstride + (static_cast<uint32_t>(e) - j * static_cast<uint32_t>(b));
-}
 
 __global__ __launch_bounds__(kHistThreads) void index_hist_kernel(
-    const int32_t* __restrict__ k_codes, int64_t n, int b, int cstride, int n_c, int64_t tile_keys,
+    const int32_t* __restrict__ k_codes, int64_t n, int b, int n_c, int64_t tile_keys,
     int64_t tiles, int32_t* __restrict__ hist) {
   extern __shared__ int32_t lds_hist[];
   const int64_t tile = blockIdx.x;
@@ -53,9 +48,9 @@ __global__ __launch_bounds__(kHistThreads) void index_hist_kernel(
   const int64_t e0 = tile * tile_keys * b;
   int64_t e1 = (tile + 1) * tile_keys * b;
   if (e1 > n * b) e1 = n * b;
-  const int32_t* kc = k_codes + bh * n * cstride;
+  const int32_t* kc = k_codes + bh * n * b;
   for (int64_t e = e0 + threadIdx.x; e < e1; e += kHistThreads) {
-    const int32_t c = kc[code_at(e, b, cstride)];
+    const int32_t c = kc[e];
     if (static_cast<uint32_t>(c) < static_cast<uint32_t>(n_c)) atomicAdd(&lds_hist[c], 1);
   }
   __syncthreads();
@@ -162,7 +157,7 @@ __global__ __launch_bounds__(kScanThreads) void index_scan_kernel(int32_t* __res
 // counts of the ranges before it, and the waves' round loops run side by side
 // (a tile's 64 rounds in one wave were a chain of memory and LDS latencies).
 __global__ __launch_bounds__(256) void index_scatter_kernel(
-    const int32_t* __restrict__ k_codes, int64_t n, int b, int cstride, int n_c, int code_bits,
+    const int32_t* __restrict__ k_codes, int64_t n, int b, int n_c, int code_bits,
     int64_t tile_keys, int64_t tiles, const int32_t* __restrict__ base,
     int32_t* __restrict__ postings) {
   extern __shared__ int32_t cursors[];
@@ -175,7 +170,7 @@ __global__ __launch_bounds__(256) void index_scatter_kernel(
   const int64_t t0 = tile * tile_keys * b;
   int64_t t1 = (tile + 1) * tile_keys * b;
   if (t1 > n * b) t1 = n * b;
-  const int32_t* kc = k_codes + bh * n * cstride;
+  const int32_t* kc = k_codes + bh * n * b;
   const int64_t per = (t1 - t0 + waves - 1) / waves;
   const int64_t e0 = min(t0 + wave * per, t1);
   const int64_t e1 = min(e0 + per, t1);
@@ -186,7 +181,7 @@ __global__ __launch_bounds__(256) void index_scatter_kernel(
     for (int x = threadIdx.x; x < waves * n_c; x += blockDim.x) cursors[x] = 0;
     __syncthreads();
     for (int64_t e = e0 + lane; e < e1; e += 64) {
-      const int32_t c = kc[code_at(e, b, cstride)];
+      const int32_t c = kc[e];
       if (static_cast<uint32_t>(c) < static_cast<uint32_t>(n_c)) atomicAdd(&cursor[c], 1);
     }
     __syncthreads();
@@ -211,7 +206,7 @@ __global__ __launch_bounds__(256) void index_scatter_kernel(
 #pragma unroll
     for (int u = 0; u < kScatterBatch; ++u) {
       const int64_t e = b0 + 64 * u + lane;
-      cb[u] = kc[code_at(e < e1 ? e : e1 - 1, b, cstride)];
+      cb[u] = kc[e < e1 ? e : e1 - 1];
     }
 #pragma unroll
     for (int u = 0; u < kScatterBatch; ++u) {
@@ -404,7 +399,7 @@ size_t hist_bytes(int64_t bh, int64_t n, int n_c);
 
 // The index kernels over entries (j, r < b) of every (batch, head); `hist`
 // is the workspace, `offsets` receives the bucket starts.
-int run_index(const int32_t* codes, int64_t bh, int64_t n, int b, int cstride, int n_c,
+int run_index(const int32_t* codes, int64_t bh, int64_t n, int b, int n_c,
               int32_t* offsets, int32_t* postings, int32_t* hist, hipStream_t st) {
   if (n * b >= (int64_t(1) << 31))
     return fail(SSA_ERR_UNSUPPORTED, "index: n * b = %lld entries per head exceed int32 positions",
@@ -416,7 +411,7 @@ int run_index(const int32_t* codes, int64_t bh, int64_t n, int b, int cstride, i
   int code_bits = 0;
   while ((1 << code_bits) < n_c) ++code_bits;
   index_hist_kernel<<<dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(bh)), kHistThreads,
-                      sizeof(int32_t) * n_c, st>>>(codes, n, b, cstride, n_c, tk, tiles, hist);
+                      sizeof(int32_t) * n_c, st>>>(codes, n, b, n_c, tk, tiles, hist);
   int s = check_launch("index_hist_kernel");
   if (s) return s;
   const int chunks = static_cast<int>(ceil_div(n_c, kScanThreads));
@@ -432,7 +427,7 @@ int run_index(const int32_t* codes, int64_t bh, int64_t n, int b, int cstride, i
   int waves = 4;
   while (waves > 1 && sizeof(int32_t) * static_cast<size_t>(n_c) * waves > 64 * 1024) waves >>= 1;
   index_scatter_kernel<<<dim3(static_cast<unsigned>(tiles), static_cast<unsigned>(bh)), 64 * waves,
-                         sizeof(int32_t) * n_c * waves, st>>>(codes, n, b, cstride, n_c, code_bits, tk,
+                         sizeof(int32_t) * n_c * waves, st>>>(codes, n, b, n_c, code_bits, tk,
                                                               tiles, hist, postings);
   return check_launch("index_scatter_kernel");
 }
@@ -449,7 +444,7 @@ size_t hist_bytes(int64_t bh, int64_t n, int n_c) {
 size_t index_ws_bytes(int64_t bh, int64_t n, int n_c) { return hist_bytes(bh, n, n_c); }
 int build_index_into(const int32_t* codes, int64_t bh, int64_t n, int b, int n_c, int32_t* offsets,
                      int32_t* postings, void* ws, hipStream_t st) {
-  return run_index(codes, bh, n, b, b, n_c, offsets, postings, static_cast<int32_t*>(ws), st);
+  return run_index(codes, bh, n, b, n_c, offsets, postings, static_cast<int32_t*>(ws), st);
 }
 
 }  // namespace ssa
@@ -483,7 +478,7 @@ extern "C" int ssa_build_index(const int32_t* k_codes, int64_t batch, int64_t n,
     fill_i32_kernel<<<dim3(static_cast<unsigned>(ceil_div(count, 256))), 256, 0, st>>>(offsets, count, 0);
     return check_launch("fill_i32_kernel");
   }
-  return run_index(k_codes, bh, n, b, b, n_c, offsets, postings, static_cast<int32_t*>(workspace), st);
+  return run_index(k_codes, bh, n, b, n_c, offsets, postings, static_cast<int32_t*>(workspace), st);
 }
 
 namespace ssa {
@@ -542,5 +537,5 @@ extern "C" int ssa_query_order(const int32_t* q_codes, int64_t batch, int64_t n,
   const int64_t rows = bh * n;
   row_min_code_kernel<<<dim3(static_cast<unsigned>(ceil_div(rows, 256))), 256, 0, st>>>(q_codes, rows, a, mins);
   if (int s = check_launch("row_min_code_kernel")) return s;
-  return run_index(mins, bh, n, 1, 1, n_c, offsets, order, hist, st);
+  return run_index(mins, bh, n, 1, n_c, offsets, order, hist, st);
 }

@@ -209,8 +209,8 @@ size_t route_vectors_tile_smem(int d) {
 
 // head_dim 64 or 128, route_dim <= 32 and a multiple of 4: the projections on the
 // fp32 matrix cores.  v_mfma_f32_32x32x2_f32 computes each product sum as fmaf
-// chains in ascending order (checked bit for bit against fmaf, denormals
-// included), so a chain of d / 2 of them over W (rows: the 32 coordinates) and x
+// chains in ascending order (bit for bit, denormals included:
+// tests/test_gpu_route_mfma.py), so a chain of d / 2 of them over W (rows: the 32 coordinates) and x
 // (columns: 32 tokens) is the canonical chain of every (token, coordinate).
 //   block   four waves, 128 tokens of one (batch, output head); a wave runs its
 //           32 tokens' heads one after the other and folds them in head order;

@@ -255,10 +255,8 @@ __device__ __forceinline__ int list_live_tiles(const uint32_t* live, int tiles, 
   return __builtin_amdgcn_readfirstlane(base);
 }
 
-// s_waitcnt encodings (gfx9): vmcnt(0) alone, lgkmcnt(0) alone; vmcnt(N) for
-// N < 16 is kWaitVmBase | N.
+// s_waitcnt encodings (gfx9): vmcnt(0) alone, lgkmcnt(0) alone.
 constexpr int kWaitVm0 = 0x0F70;
-constexpr int kWaitVmBase = 0x0F70;
 constexpr int kWaitLgkm0 = 0xC07F;
 
 // Which chunks (kMfChunk index slots each) of a row hold a key to attend.  A

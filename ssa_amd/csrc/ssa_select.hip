@@ -599,7 +599,7 @@ __device__ __forceinline__ void sort_slots_desc(uint64_t* keys, int lane) {
 // lane l's own key as column l % 4 of block l / 4 and the group's query head l % 4 as
 // row, so each lane ends with its key's dot products with four heads, and a chain of
 // D of them over ascending dimensions is the canonical fmaf chain, bit for bit
-// (checked against fmaf, denormals included).  That is half the issue time of the
+// (denormals included: tests/test_gpu_sort_rows.py, test_gpu_select_few.py).  That is half the issue time of the
 // vector ALU's chains and leaves it to the bf16 conversions.
 // qs: the query rows in LDS as fp32, row stride kQsRow (rows past g zero).
 template <int D>
@@ -651,7 +651,8 @@ __device__ __forceinline__ float score_of_acc(const SelParams& p, const floatx4_
 // load instruction moves eight whole cache lines (a lane reading its own row in
 // 16-byte pieces touches 64 of them per instruction).  A step's rows go on to
 // registers at once and the one buffer takes the next step's while they are
-// multiplied: 10 KB of LDS a wave, 15 waves a CU.  Segments are XOR-swizzled by row / 2, so the
+// multiplied: 10 KB of LDS a wave and 15 waves a CU
+// up to four heads a group at D = 128 (16 heads: 17 KB, 9 waves).  Segments are XOR-swizzled by row / 2, so the
 // lanes' reads of their own rows hit distinct banks.
 // n = 32768, 32/8 heads, d = 128, k = 512: 1.78 ms against 2.88 ms with the
 // vector-ALU chains of select_sort_kernel on rows read lane by lane (81% of the time
