@@ -2244,6 +2244,22 @@ constexpr int64_t kTileRows = 65536;
 // ... and up to which a block takes 16 rows and not 32, which reads the codebook twice
 // as often: 2048 rows of 2 heads 44 against 48 us, 1024 rows of 8 heads 71 against 61.
 constexpr int64_t kTileNarrowRows = 8192;
+// Whether `tasks` tasks of `rows` rows in all take it.  With 32 rows a block a row has two
+// maxima a lane, and a small codebook leaves each only a few codes: the bound lies low,
+// lists overrun and rows run exhaustively (N_c 128, 16 codes, 65536 rows: 52 -> 457 us).
+// A codebook that fits the list cannot overrun it.  256-row blocks / this, us, d_s = 32:
+//   one task    rows 16384:  N_c 64, 8 codes 35 / 31;   N_c 128, 16 codes 52 / 140;  N_c 256, 16 codes 58 / 65
+//               rows 32768:  N_c 64, 8 codes 35 / 56, 32 codes 194 / 79;   N_c 256, 32 codes 187 / 470
+//               rows 49152:  N_c 512, 16 codes 65 / 50; N_c 16384, 4 codes 207 / 206
+//               rows 65536:  N_c 1024, 1 code 35 / 41;  16 codes 73 / 75;  32 codes 172 / 138
+//   two (a, 4)  rows 32768:  N_c 128, a = 8 98 / 46, a = 16 93 / 148;  N_c 256, a = 16 101 / 71, a = 32 254 / 278
+//               rows 65536:  N_c 64, a = 16 121 / 91;   N_c 256, a = 16 103 / 121 - 168
+inline bool topk_tile_ok(int64_t rows, int tasks, int top, int n_c) {
+  if (rows <= kTileNarrowRows) return true;
+  const bool tight = n_c <= kTileCap || n_c >= 32 * top || n_c >= 512;
+  if (tasks == 2) return rows <= (tight ? kTileRows : n_c >= 16 * top ? 49152 : 0);
+  return tight && rows <= (top > 16 ? kTileRows : n_c < 512 ? 24576 : 49152);
+}
 
 bool mfma_path_ok(int top, int d_s, int n_c) { return top <= 32 && d_s <= 32 && d_s % 4 == 0 && n_c <= 65535; }
 
@@ -2360,7 +2376,7 @@ int launch_code_topk_w(const float* xhat, int64_t batch, int h, int64_t rows, co
     FewTopk none{};
     return launch_topk_few(t0, none, h, chat, n_c, d_s, temperature, st);
   }
-  if (batch * h * rows <= kTileRows) {
+  if (topk_tile_ok(batch * h * rows, 1, top, n_c)) {
     const FewTopk t0{xhat, rows, batch * h * rows, top, codes};
     return launch_topk_tile(t0, FewTopk{}, h, chat, n_c, d_s, temperature, w, st);
   }
@@ -2572,7 +2588,8 @@ extern "C" int ssa_route_codes(const void* q, const void* k, int dtype, int64_t 
       return st;
   }
   const int64_t rows = batch * h_kv * n;
-  if (rows > kFewTopkRows && 2 * rows <= kTileRows && mfma_path_ok(a, d_s, n_c) && mfma_path_ok(b, d_s, n_c)) {
+  if (rows > kFewTopkRows && topk_tile_ok(2 * rows, 2, std::max(a, b), n_c) && mfma_path_ok(a, d_s, n_c) &&
+      mfma_path_ok(b, d_s, n_c)) {
     const TopkWorkspace w = carve_topk(tws, h_kv, n_c);
     if ((st = launch_codebook_prep(codebook, chat, h_kv, n_c, d_s, w, s))) return st;
     const FewTopk tq{qhat, n, rows, a, q_codes}, tk{khat, n, rows, b, k_codes};

@@ -78,3 +78,27 @@ def test_codebook_normalized_with_its_copy(dev, orc, shift, d_s):
     for got, x, top in zip(kernels.route_codes(q.to(dev), k.to(dev), w.to(dev), w.to(dev), cbd, 16, 4), (q, k), (16, 4)):
         ref = orc.code_topk(orc.route_vectors(x[0].numpy(), w.numpy(), 1), chat, top)
         np.testing.assert_array_equal(got[0].cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("h,rows,n_c,top", [(2, 4096, 128, 16), (2, 4097, 128, 16), (2, 4097, 112, 16), (2, 4097, 113, 16),
+                                            (3, 8192, 256, 8), (3, 8193, 256, 8), (3, 16384, 512, 20), (3, 16385, 512, 16),
+                                            (3, 16385, 512, 17), (3, 16385, 64, 32)])
+def test_code_tiles_on_both_sides_of_their_rule(dev, h, rows, n_c, top):
+    """By the rows, and with a small codebook by what its lists would overrun."""
+    from ssa_amd import kernels
+
+    x, c = (t.to(dev) for t in _inputs(1, h, rows, n_c, 32, 51))
+    assert torch.equal(kernels.code_topk(x, c, top), kernels.code_topk(x, c, top, exhaustive=True))
+
+
+@pytest.mark.parametrize("rows,n_c,a", [(2049, 128, 16), (2049, 128, 8), (2049, 256, 32), (3072, 256, 16), (3073, 256, 16)])
+def test_route_codes_on_both_sides_of_the_tiles_rule(dev, rows, n_c, a):
+    from ssa_amd import kernels
+
+    h, d, d_s = 8, 64, 32
+    q, k = randn((1, rows, h, d), 55).to(dev), randn((1, rows, h, d), 56).to(dev)
+    w, cb = randn((d_s, d), 57).to(dev), randn((h, n_c, d_s), 58).to(dev)
+    chat = kernels.normalize_rows(cb)
+    for got, x, top in zip(kernels.route_codes(q, k, w, w, cb, a, 4), (q, k), (a, 4)):
+        ref = kernels.code_topk(kernels.route_vectors(x, w, 1), chat, top, exhaustive=True)
+        assert torch.equal(got, ref)
