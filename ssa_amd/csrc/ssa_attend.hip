@@ -1739,7 +1739,8 @@ __global__ __launch_bounds__(64 * kDnWaves, 2) void dense_f32_kernel(AttParams p
 //            2 kv heads, g = 4:  n = 2048, k = 512: 338 / 235;  n = 16384, k = 4096: 21.8 / 14.6 ms
 //            8 kv heads, g = 1, n = 2048, k = 256: 1 row 44 / 71;  128 rows 50 / 94;  512 rows 182 / 95
 // Two 16-query tiles a block at d = 64 once that leaves 512 blocks (2 waves a
-// SIMD); at d = 128 two do not fit the registers.
+// SIMD); at d = 128 two do not fit the registers (one takes all 256 and spills 4: 20
+// bytes of scratch a lane).
 constexpr int kDnKeysPerSlot = 16;
 constexpr int64_t kDnTwoTiles = 32 * 512;  // query vectors
 

@@ -19,7 +19,7 @@ def _case(n, h_kv, g, d, k, seed):
 
 
 @pytest.mark.parametrize("d,g,h_kv,n,k,causal,i64", [
-    (64, 1, 2, 1999, 300, False, True),    # 16 rows a block, four key windows
+    (64, 1, 2, 1999, 300, False, True),    # 16 rows a block, two key windows
     (64, 3, 2, 331, 70, True, False),      # 15 of 16 query vectors used
     (64, 4, 4, 1100, 300, True, True),     # two query tiles a block
     (128, 5, 1, 257, 100, True, True),
